@@ -432,7 +432,7 @@ int mk2_layer_step_is_fused(const mk2_front_shape* shape, int expert_fmt);
  *   normed[r]    = bf16(x[r] * rsqrt(mean(x[r]^2) + eps) * g_norm)
  *   logits[r][v] = f32(bf16(normed[r] . w_head[v]))   (bf16 as the reference gathers)
  * w_head is SGLang's LM head as loaded, bf16 [vocab_rows][hidden] row-major, read in
- * place.  No workspace.  More than 16 rows stream the LM head twice. */
+ * place, once.  No workspace. */
 typedef struct mk2_tail_args {
   int rows;             /* 1..32 */
   int hidden;           /* multiple of 1024 in [2048, 8192] */

@@ -85,6 +85,24 @@ def test_tail_other_shapes(hidden, vocab_rows, rows):
     _check(cfg, ns, logits, normed)
 
 
+@pytest.mark.parametrize("hidden, vocab_rows, rows", [(2048, 4103, 17), (3072, 1, 32), (4096, 5000, 24), (5120, 4111, 31),
+                                                      (6144, 19360, 32), (6144, 300, 17), (7168, 4097, 18), (8192, 2050, 32)])
+def test_tail_above_16_rows_in_one_pass(hidden, vocab_rows, rows):
+    """Above 16 rows one pass over the LM head serves two column groups: the bits of the
+    rows taken in two calls, at every hidden size's operand placement (registers, or part
+    of the second group in LDS), with partial last tiles and fewer vocab rows than CUs."""
+    from sgl_amd_mono.k2 import config as C
+    from sgl_amd_mono.k2.ops import TailOp
+
+    cfg = C.TailConfig(hidden=hidden, vocab_rows=vocab_rows)
+    ns, logits, normed = _run(cfg, rows, seed=hidden + rows)
+    if vocab_rows > 1:
+        _check(cfg, ns, logits, normed)
+    for a, b in ((0, 16), (16, rows)):
+        lo, no = TailOp(cfg, ns.g_norm, ns.w_head, b - a, device=_dev())(ns.x[a:b].contiguous())
+        assert torch.equal(cpu(lo), logits[a:b]) and torch.equal(cpu(no).float(), normed[a:b])
+
+
 def test_tail_repeats_bit_identical():
     from sgl_amd_mono.k2 import config as C, synth
     from sgl_amd_mono.k2.ops import TailOp
