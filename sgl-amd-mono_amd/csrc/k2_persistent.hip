@@ -76,7 +76,7 @@ MK2_DEV void k2_stamp(const K2Dev& p, int i) {
 union K2Lds {
   IdxScoreLds score;
   TopkLds topk;
-  MlaSplitLds split;
+  MlaSplitLds split[2];  // the workgroup's, or its two halves'
   MlaMergeLds merge;
   struct {
     float red[(K2_NT / 64) * 8 * 64 * 4];  // NW * 2 * CT * NCG * 256, CT * NCG <= 4
@@ -95,6 +95,11 @@ union K2Lds {
 static_assert(sizeof(FrontLds) <= sizeof(TopkLds), "the front's LDS fits the layer's union as it is");
 
 MK2_DEV int* k2_ctr(const K2Dev& p, int line) { return p.sync + line * SY_LINE; }
+
+// one finished task onto a counter, by a thread whose workgroup's stores have drained
+MK2_DEV void k2_count(const K2Dev& p, int line) {
+  __hip_atomic_fetch_add(k2_ctr(p, line), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // publish n finished tasks on counter `line` (sub-counter t mod lanes): every thread's
 // stores drained, then one increment
@@ -163,6 +168,27 @@ MK2_DEV bool k2_wait(const K2Dev& p, int* seen, int line, int target, int stamp 
   __syncthreads();  // the flag is read before the next wait can write it
   if (threadIdx.x == 0 && ok) seen[line] = v;
   return ok;
+}
+
+// The split tasks of workgroup w (in the stage's rotation), counted out by row: up to 16
+// rows every G-th, one after another (one or two of 2048 keys a row); above, an equal run
+// of consecutive tasks for each of the workgroup's halves, two at once (32 rows, the whole
+// MLA block: 55.0 -> 42.4 us, 27 rows 48.3 -> 42.7).  One form a kernel: with both in it
+// the 8-row layer, whose code runs once, was 2-3 us slower.
+template <int NCG, typename Mark = NoMark>
+MK2_DEV bool k2_splits(const K2Dev& p, K2Lds& S, int w, const TagPoll& tp, Mark mark = Mark()) {
+  const int G = gridDim.x, ns = p.mla.nsplit, n = p.rows * ns;
+  auto done = [&](int t) { k2_count(p, SY_SPLIT + t / ns); };
+  if constexpr (NCG == 1) {
+    for (int t = w; t < n; t += G)
+      if (!mla_split_tasks<K2_NT, false>(p.mla, t, t + 1, 1, S.split, tp, done, [&](int i) { if (t < G) mark(i); }))
+        return false;
+    return true;
+  }
+  auto first = [&](int u) { return u * n / (2 * G); };  // n <= 32 * 1024, u <= 2 G
+  const int u = 2 * w + __builtin_amdgcn_readfirstlane(threadIdx.x / (K2_NT / 2));
+  const int iters = max(first(2 * w + 1) - first(2 * w), first(2 * w + 2) - first(2 * w + 1));
+  return mla_split_tasks<K2_NT / 2, true>(p.mla, first(u), first(u + 1), iters, S.split, tp, done, mark);
 }
 
 // The up/gate tasks (up_total of them: the shared expert's chunks, then the routed
@@ -330,15 +356,9 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
     // ---- sparse-MLA splits
     k2_stamp(p, 3 * st);
     const int ns = p.mla.nsplit;
-    K2_TASKS(t, R * ns) {
-      const int r = t / ns;
-      // the split polls its 64 entries of the tagged list: it starts as soon as they are
-      // out (most come from the slices, ahead of the row's select)
-      const int stamp = t < G ? 3 * st + 1 : -1;
-      if (!mla_split<K2_NT>(p.mla, r, t % ns, S.split, tp, [&](int) { if (stamp >= 0) k2_stamp(p, stamp); }))
-        return;
-      k2_signal(p, SY_SPLIT + r);
-    }
+    // a split polls its 64 entries of the tagged list: it starts as soon as they are out
+    // (most come from the slices, ahead of the row's select)
+    if (!k2_splits<NCG>(p, S, (b - base % G + G) % G, tp, [&](int) { k2_stamp(p, 3 * st + 1); })) return;
     K2_NEXT(R * ns);
     k2_stamp(p, 3 * st++ + 2);
     // ---- merge of the splits + W_UV, per (group of mrg rows, head, half of the head's
@@ -616,10 +636,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_block(K2Dev p) {
     } else if constexpr (BLK == K2_BLOCK_MLA) {
       // splits (the given positions), merge + W_UV, W_o + residual: as the layer's
       const int ns = p.mla.nsplit;
-      K2_TASKS(t, R * ns) {
-        if (!mla_split<K2_NT>(p.mla, t / ns, t % ns, S.split, tp)) return;
-        k2_signal(p, SY_SPLIT + t / ns);
-      }
+      if (!k2_splits<NCG>(p, S, b, tp)) return;
       K2_NEXT(R * ns);
       const int mrg = mla_merge_rows(R, G), nmt = 2 * MLA_HEADS * ((R + mrg - 1) / mrg);
       K2_TASKS(t, nmt) {

@@ -22,6 +22,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef uint16_t bf16_t;  // storage type of bf16 in memory
@@ -300,6 +301,16 @@ MK2_DEV void st_dev_16(void* p, uint4 v) {
   MK2_DEV_ST(uint64_t, p, ((uint64_t)v.y << 32) | v.x);
   MK2_DEV_ST(uint64_t, (uint64_t*)p + 1, ((uint64_t)v.w << 32) | v.z);
 }
+// A workgroup's output block (a uniform base) written in whole 16-byte device-coherent
+// stores: as two 8-byte stores (st_dev_16) each of a wave's instructions fills every other
+// half of the lines it writes.
+struct DevOut {
+  __amdgpu_buffer_rsrc_t rs;
+  MK2_DEV DevOut(void* base, int bytes) : rs(__builtin_amdgcn_make_buffer_rsrc(base, (short)0, bytes, 0x00020000)) {}
+  MK2_DEV void st16(int at, uint4 v) const {
+    __builtin_amdgcn_raw_buffer_store_b128(i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w}, rs, at, 0, 16 /* sc1 */);
+  }
+};
 // the dependency wait a stage runs after issuing the loads of its static weights (the
 // persistent launch waits on a counter there; a stand-alone kernel has nothing to wait
 // for)

@@ -10,7 +10,8 @@ namespace mk2 {
 
 __global__ __launch_bounds__(MLA_NT) void k_mla_split(MlaDev p) {
   __shared__ MlaSplitLds L;
-  mla_split<MLA_NT>(p, blockIdx.y, blockIdx.x, L, TagPoll{0u, 0, nullptr});
+  const int t = blockIdx.y * p.nsplit + blockIdx.x;
+  mla_split_tasks<MLA_NT, false>(p, t, t + 1, 1, &L, TagPoll{0u, 0, nullptr}, [](int) {});
 }
 // merge + W_UV and W_o run 512 threads, as in the persistent layer kernel: the same
 // waves split the same sums, so both paths give the same bits

@@ -2,9 +2,8 @@
 // rows, the merge of the splits, W_UV, and W_o with the residual.
 //
 // split task (row r, split s): 64 selected positions -> page table -> 576-byte E4M3
-// rows, gathered with 16-byte loads into LDS twice: row-major (the QK operand) and,
-// for the first 512 dims, transposed to [dim][key] (the PV operand, 8 keys a lane
-// read).  S = q . k on bf16 MFMA (E4M3 widens exactly), x (scale_k * sm_scale); a
+// rows, gathered with 16-byte loads into LDS row-major: the QK operand as it lies, the PV
+// operand (8 keys of a dim a lane) by transposing LDS reads.  S = q . k on bf16 MFMA (E4M3 widens exactly), x (scale_k * sm_scale); a
 // split-local softmax per head; P' = p * scale_k rounded to bf16; O = P' V on bf16
 // MFMA.  The split writes O (unnormalized), its max m and sum l.
 // merge task (up to 4 rows, head h, half): exact combination of each row's splits ->
@@ -19,13 +18,10 @@ constexpr int MLA_D = 576;        // latent 512 + rope 64
 constexpr int MLA_LAT = 512;
 constexpr int MLA_HEADS = 16;
 constexpr int MLA_SPLIT = 64;     // keys a split task
-constexpr int MLA_KROW = 584;     // LDS row stride of the gathered rows (bytes)
-constexpr int MLA_VROW = 72;      // LDS row stride of the transposed latent (bytes)
-// In the transposed latent, dim d's 4-key word w sits at word w ^ mla_vswz(d): the
-// gather writes one word of 16 consecutive dims a lane, and without the swizzle all
-// lanes of a store would hit one bank (16 rows of 18 words is 0 mod 32).  The swizzle
-// is even, so the two words of an aligned 8-key read stay an aligned pair.
-MK2_DEV int mla_vswz(int d) { return 2 * ((d >> 4) & 7); }
+// LDS row stride of the gathered rows (bytes): 16-byte pieces, and 148 words, so that the
+// QK reads (8 bytes of each of 16 rows) and the transposing PV reads (16 bytes of each of 8
+// rows) fall in distinct banks
+constexpr int MLA_KROW = 592;
 constexpr int MLA_NT = 256;
 
 struct MlaDev {
@@ -51,214 +47,260 @@ struct MlaDev {
   float* ssp;            // optional [rows][hidden/16]: sums of squares of out over 16 columns
 };
 
-struct MlaSplitLds {
+struct alignas(16) MlaSplitLds {
   uint8_t k[MLA_SPLIT * MLA_KROW];       // gathered rows, row-major
-  uint8_t vt[MLA_LAT * MLA_VROW];        // latent dims transposed: [dim][key]
   bf16_t p[MLA_HEADS * (MLA_SPLIT + 8)]; // P' [head][key]
-  int row[MLA_SPLIT + 1];                // cache row of each key (-1: unused); [64]: a poll gave up
+  int row[2][MLA_SPLIT];                 // by task parity: cache row of each key (-1: unused)
   float sc[MLA_SPLIT];                   // per-key scale * sm_scale
   float kscale[MLA_SPLIT];
-  float red[4][MLA_HEADS];
+  alignas(16) float red[4][MLA_HEADS];   // by wave: its keys' maxima by head
+  alignas(16) float suml[4][MLA_HEADS];  // and its sums
+  int bad;                               // a poll gave up
 };
+typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
+// PV's operand from the row-major E4M3 rows: 8 keys (rows of `k`) x 16 dims a 16-lane group,
+// lane i of which gets dim d0 + i of keys key0 .. key0 + 7 (lanes 2j, 2j + 1 address key j's
+// two 8-byte halves; the read transposes)
+MK2_DEV uint2 lds_read_keys8(const uint8_t* k, int key0, int d0, int i) {
+  const i32x2 r = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+      (lds_i32x2*)(k + (key0 + (i >> 1)) * MLA_KROW + d0 + 8 * (i & 1)));
+  return make_uint2((uint32_t)r.x, (uint32_t)r.y);
+}
 
 // ---------------------------------------------------------------- stage: split
-// NT = 256 or 512: waves 0-3 run QK and the softmax (16 keys each), every wave
-// gathers and takes a share of the PV dim tiles.
-template <int NT, typename Mark = NoMark>
-MK2_DEV bool mla_split(const MlaDev& p, int r, int s, MlaSplitLds& L, const TagPoll& tp, Mark mark = Mark()) {
+// The split tasks t0 .. t1 - 1 (task t: row t / nsplit, split t % nsplit) of one worker: NT =
+// 256 or 512 threads, waves 0-3 of which run QK and the softmax (16 keys each), every wave
+// gathering and taking a share of the PV dim tiles.  A worker is the workgroup, or (HALF)
+// its half threadIdx.x / NT with LDS of its own; the halves keep step, `iters` being the
+// larger half's number of tasks.
+//
+// Without HALF a worker runs one task.  With several tasks a workgroup, QK and the softmax,
+// chains of latencies on four waves, leave the other four idle: the halves run two tasks
+// at once, neighbours of one row, so that the q operands stay.  A half's tasks also
+// overlap: while one computes, the next one's rows are in flight into registers, and on
+// its last wave the cache rows of the one after it and the positions of the third.  A
+// task's partials are counted out (`done(t)`, by one thread) once the next one's rows have
+// arrived, where waiting for the stores costs nothing; the last task's right away.
+template <int NT, bool HALF, typename Done, typename Mark = NoMark>
+MK2_DEV bool mla_split_tasks(const MlaDev& p, int t0, int t1, int iters, MlaSplitLds* LS, const TagPoll& tp, Done done,
+                             Mark mark = Mark()) {
   constexpr int NW = NT / 64;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, c16 = lane & 15;
+  const int tid = threadIdx.x % NT, lane = tid & 63, wave = tid >> 6, g = lane >> 4, c16 = lane & 15;
   const bool qk_wave = wave < 4;
-  const int* selr = p.sel + (size_t)r * p.topk + s * MLA_SPLIT;
-  const int* ptr = p.pt + (size_t)p.req[r] * p.stride;
-  // q operands for this wave's QK: head c16, dims 8g + 32ks .. +7.  Wave 0 loads its
-  // own behind the gather: ahead of its list poll and page-table read they would hold
-  // both up (a wave's loads complete in order)
+  if (iters <= 0) return true;
+  MlaSplitLds& L = LS[HALF ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0];
+  auto failed = [&] { return LS[0].bad != 0 || (HALF && LS[1].bad != 0); };
+  // q operands for this wave's QK: head c16, dims 8g + 32ks .. +7
   bf16x8 qa[18];
-  const bf16_t* qr = p.q + ((size_t)r * MLA_HEADS + c16) * MLA_D + 8 * g;
-  auto load_q = [&] {
+  auto load_q = [&](int r) {
+    const bf16_t* qr = p.q + ((size_t)r * MLA_HEADS + c16) * MLA_D + 8 * g;
 #pragma unroll
     for (int ks = 0; ks < 18; ++ks) qa[ks] = __builtin_bit_cast(bf16x8, *(const uint4*)(qr + 32 * ks));
   };
-  if (qk_wave && wave != 0) load_q();
-  // resolve the 64 positions to cache rows (one dependent round); the rows' scales
-  // are loaded with the rows below.  A tagged list is polled here, one entry a lane of
-  // wave 0: the split starts as soon as its own 64 entries are out.
-  if (tid < MLA_SPLIT) {
-    int pos;
-    bool bad = false;
+  // one wave: a task's 64 positions, an entry a lane, as words of the list (a tagged list's
+  // are checked, and polled where they are not out yet: the task starts as soon as its own
+  // 64 entries are), then the cache row of a position
+  auto list_at = [&](int t) {
+    return (size_t)(t / p.nsplit) * p.topk + (t % p.nsplit) * MLA_SPLIT + lane;
+  };
+  auto list_word = [&](int t) -> uint64_t {
+    return p.tsel ? ld_pair(p.tsel + list_at(t)) : (uint64_t)(uint32_t)ldp_i32(p.sel + list_at(t));
+  };
+  auto list_poll = [&](int t, uint64_t w, bool* bad) {
     if (p.tsel) {
-      const uint64_t* src = p.tsel + (size_t)r * p.topk + s * MLA_SPLIT + tid;
-      uint64_t w = ld_pair(src);
+      const uint64_t* src = p.tsel + list_at(t);
       WaitClock wc;
       for (int polls = 1;; polls += 2) {  // two polls in flight
         const uint64_t w1 = ld_pair(src);
-        if (poll_done(pair_ready(w, tp), polls, wc, tp, &bad)) break;
+        if (poll_done(pair_ready(w, tp), polls, wc, tp, bad)) break;
         w = ld_pair(src);
-        if (poll_done(pair_ready(w1, tp), polls + 1, wc, tp, &bad)) {
+        if (poll_done(pair_ready(w1, tp), polls + 1, wc, tp, bad)) {
           w = w1;
           break;
         }
       }
-      pos = (int)pair_value(w);
-    } else {
-      pos = ldp_i32(selr + tid);
     }
-    if (tid == 0) L.row[MLA_SPLIT] = bad;  // wave-uniform
-    int row = -1;
-    if (pos >= 0 && pos < p.stride * 64) row = ptr[pos >> 6] * 64 + (pos & 63);
-    L.row[tid] = row;
-  }
-  if (tid == 0) mark(0);
-  __syncthreads();
-  if (L.row[MLA_SPLIT]) return false;
+    return (int)pair_value(w);
+  };
+  // (the page's load has no use here to wait for)
+  auto on_page = [&](int pos) { return pos >= 0 && pos < p.stride * 64; };
+  auto page_of = [&](int t, int pos) {
+    return p.pt[(size_t)p.req[t / p.nsplit] * p.stride + (on_page(pos) ? pos >> 6 : 0)];
+  };
+  auto cache_row = [&](int pos, int page) { return on_page(pos) ? page * 64 + (pos & 63) : -1; };
+  // gather: 16-byte piece i % 36 of key i / 36; every load of a thread is issued at once,
+  // the rows' scales ahead of them
+  constexpr int PIECES = MLA_SPLIT * (MLA_D / 16), PPT = (PIECES + NT - 1) / NT;
+  uint4 v[PPT];
   float ksc = 0.f;
-  if (tid < MLA_SPLIT) {
-    const int row = L.row[tid];
-    ksc = row < 0 ? 0.f : (p.kv_scale ? p.kv_scale[row] : 1.f);
-  }
-  // gather: job = (4-key group kg, 16-byte dim chunk dc), 16 x 36 jobs; every load of
-  // a thread is issued before the first LDS store
-  constexpr int JOBS = 16 * 36, JPT = (JOBS + NT - 1) / NT;
-  uint4 v[JPT][4];
+  auto gather = [&](const int* row) {
+    if (tid < MLA_SPLIT) ksc = row[tid] < 0 ? 0.f : (p.kv_scale ? p.kv_scale[row[tid]] : 1.f);
 #pragma unroll
-  for (int it = 0; it < JPT; ++it) {
-    const int job = tid + it * NT;
-    const int kg = job / 36, dc = job % 36;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int row = job < JOBS ? L.row[kg * 4 + j] : -1;
-      v[it][j] = row >= 0 ? ld_stream16(p.kv + (size_t)row * MLA_D + dc * 16) : make_uint4(0, 0, 0, 0);
+    for (int it = 0; it < PPT; ++it) {
+      const int i = tid + it * NT;
+      const int rw = i < PIECES ? row[i / 36] : -1;
+      v[it] = rw >= 0 ? ld_stream16(p.kv + (size_t)rw * MLA_D + i % 36 * 16) : make_uint4(0, 0, 0, 0);
     }
-  }
-  if (wave == 0) load_q();
-  if (tid < MLA_SPLIT) {
-    L.kscale[tid] = ksc;
-    L.sc[tid] = ksc * p.sm_scale;
-  }
-#pragma unroll
-  for (int it = 0; it < JPT; ++it) {
-    const int job = tid + it * NT;
-    if (job >= JOBS) break;
-    const int kg = job / 36, dc = job % 36;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      uint8_t* dst = L.k + (kg * 4 + j) * MLA_KROW + dc * 16;
-      *(uint2*)dst = make_uint2(v[it][j].x, v[it][j].y);
-      *(uint2*)(dst + 8) = make_uint2(v[it][j].z, v[it][j].w);
+  };
+  // the first task's rows, and the second's positions beside them.  Wave 0 loads its q
+  // behind the gather: ahead of its list poll and page-table read they would hold both up
+  // (a wave's loads complete in order)
+  const bool any = t0 < t1;
+  if (any && qk_wave && wave != 0) load_q(t0 / p.nsplit);
+  const bool ahead = HALF && wave == NW - 1 && t0 + 1 < t1;  // the wave that resolves later tasks
+  uint64_t aw = 0;           // the list words it looks at next
+  int apos = -1, apage = 0;  // positions and pages of the task before those
+  bool abad = false;
+  if (wave == 0) {
+    bool bad = false;
+    if (any) {
+      const int pos = list_poll(t0, list_word(t0), &bad);
+      L.row[0][lane] = cache_row(pos, page_of(t0, pos));
     }
-    if (dc < 32) {
-      // transpose 4 keys x 16 dims of bytes -> 16 words of 4 keys
+    if (lane == 0) L.bad = bad;  // wave-uniform
+  }
+  if (ahead) aw = list_word(t0 + 1);
+  if (threadIdx.x == 0) mark(0);
+  __syncthreads();
+  if (failed()) return false;
+  if (ahead) {
+    apos = list_poll(t0 + 1, aw, &abad);
+    apage = page_of(t0 + 1, apos);
+    if (t0 + 2 < t1) aw = list_word(t0 + 2);
+  }
+  if (any) {
+    gather(L.row[0]);
+    if (wave == 0) load_q(t0 / p.nsplit);
+  }
+  for (int i0 = 0, t = t0, par = 0; i0 < (HALF ? iters : 1); ++i0, ++t, par ^= 1) {
+    const int r = t / p.nsplit, s = t % p.nsplit;
+    const int* row = L.row[par];
+    const bool have = t < t1, more = HALF && t + 1 < t1;
+    if (have) {
+      if (tid < MLA_SPLIT) {
+        L.kscale[tid] = ksc;
+        L.sc[tid] = ksc * p.sm_scale;
+      }
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint32_t w0 = ((const uint32_t*)&v[it][0])[q], w1 = ((const uint32_t*)&v[it][1])[q];
-        const uint32_t w2 = ((const uint32_t*)&v[it][2])[q], w3 = ((const uint32_t*)&v[it][3])[q];
-        const uint32_t lo01 = __builtin_amdgcn_perm(w1, w0, 0x05010400u);  // b0 of w0,w1 | b1 of w0,w1
-        const uint32_t hi01 = __builtin_amdgcn_perm(w1, w0, 0x07030602u);  // b2.. | b3..
-        const uint32_t lo23 = __builtin_amdgcn_perm(w3, w2, 0x05010400u);
-        const uint32_t hi23 = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
-        const int d = dc * 16 + q * 4;
-        const int w = (kg ^ mla_vswz(d)) * 4;  // the four dims share d >> 4
-        *(uint32_t*)(L.vt + (d + 0) * MLA_VROW + w) = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-        *(uint32_t*)(L.vt + (d + 1) * MLA_VROW + w) = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-        *(uint32_t*)(L.vt + (d + 2) * MLA_VROW + w) = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-        *(uint32_t*)(L.vt + (d + 3) * MLA_VROW + w) = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+      for (int it = 0; it < PPT; ++it) {
+        const int i = tid + it * NT;
+        if (i < PIECES) *(uint4*)(L.k + i / 36 * MLA_KROW + i % 36 * 16) = v[it];
       }
     }
-  }
-  __syncthreads();
-  // QK: wave w < 4 takes keys 16w .. 16w+15 as the MFMA columns
-  const int key = (wave & 3) * 16 + c16;
-  const bool valid = L.row[key] >= 0;
-  float sv[4], m[4];
-  if (qk_wave) {
-    // every LDS read first, then two interleaved accumulator chains
-    const uint8_t* krow = L.k + key * MLA_KROW + 8 * g;
-    uint2 kw[18];
-#pragma unroll
-    for (int ks = 0; ks < 18; ++ks) kw[ks] = *(const uint2*)(krow + 32 * ks);
-    f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < 18; ks += 2) {
-      acc0 = mfma_bf16(qa[ks], e4m3x8_to_bf16(kw[ks].x, kw[ks].y), acc0);
-      acc1 = mfma_bf16(qa[ks + 1], e4m3x8_to_bf16(kw[ks + 1].x, kw[ks + 1].y), acc1);
+    if (ahead && more) {  // the next task's rows
+      L.row[par ^ 1][lane] = cache_row(apos, apage);
+      if (lane == 0 && abad) L.bad = 1;
     }
-    const f32x4 acc = acc0 + acc1;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sv[i] = valid ? acc[i] * L.sc[key] : -INFINITY;
-    // split-local softmax per head (heads 4g + i)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float mx = row16_max(sv[i]);
-      if (c16 == 0) L.red[wave][4 * g + i] = mx;
+    if (HALF && i0) drain_memory();  // the previous task's partials are out
+    __syncthreads();
+    if (HALF && i0 && tid == 0 && t <= t1 && any) done(t - 1);
+    if (HALF && failed()) return false;
+    if (more) {
+      // the pages of the task after it and the list words of the one after that go out ahead
+      // of the gather: behind it they would hold this wave, and so the barriers, to its end
+      if (ahead && t + 2 < t1) {
+        apos = list_poll(t + 2, aw, &abad);
+        apage = page_of(t + 2, apos);
+        if (t + 3 < t1) aw = list_word(t + 3);
+      }
+      gather(L.row[par ^ 1]);
     }
-  }
-  __syncthreads();
-  float ls[4];
-  if (qk_wave) {
+    // QK: wave w < 4 takes keys 16w .. 16w+15 as the MFMA columns
+    const int key = (wave & 3) * 16 + c16;
+    const bool valid = have && row[key] >= 0;
+    float sv[4], m[4];
+    if (have && qk_wave) {
+      // every LDS read first, then two interleaved accumulator chains
+      const uint8_t* krow = L.k + key * MLA_KROW + 8 * g;
+      uint2 kw[18];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int hd = 4 * g + i;
-      m[i] = fmaxf(fmaxf(L.red[0][hd], L.red[1][hd]), fmaxf(L.red[2][hd], L.red[3][hd]));
-      const float pe = (valid && m[i] != -INFINITY) ? expf(sv[i] - m[i]) : 0.f;
-      ls[i] = row16_sum(pe);
-      L.p[hd * (MLA_SPLIT + 8) + key] = f32_to_bf16(pe * L.kscale[key]);
+      for (int ks = 0; ks < 18; ++ks) kw[ks] = *(const uint2*)(krow + 32 * ks);
+      f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 18; ks += 2) {
+        acc0 = mfma_bf16(qa[ks], e4m3x8_to_bf16(kw[ks].x, kw[ks].y), acc0);
+        acc1 = mfma_bf16(qa[ks + 1], e4m3x8_to_bf16(kw[ks + 1].x, kw[ks + 1].y), acc1);
+      }
+      const f32x4 acc = acc0 + acc1;
+      // split-local softmax per head (heads 4g + i): the wave's maxima, one 16-byte store a row
+      f32x4 mx;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sv[i] = valid ? acc[i] * L.sc[key] : -INFINITY;
+        mx[i] = row16_max(sv[i]);
+      }
+      if (c16 == 0) *(f32x4*)&L.red[wave][4 * g] = mx;
+      if (more && (t + 1) / p.nsplit != r) load_q(r + 1);
     }
-  }
-  __syncthreads();
-  if (qk_wave && c16 == 0) {
+    __syncthreads();
+    if (have && qk_wave) {
+      // every LDS read ahead of the first write, the four heads side by side: one head after
+      // another, each behind its own reads, took twice as long
+      f32x4 rd[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) L.red[wave][4 * g + i] = ls[i];
-  }
-  __syncthreads();
-  float* mlo = p.part_ml + (((size_t)r * p.nsplit + s) * MLA_HEADS) * 2;
-  if (wave == 0 && c16 == 0) {
+      for (int w = 0; w < 4; ++w) rd[w] = *(const f32x4*)&L.red[w][4 * g];
+      const float ksk = L.kscale[key];
+      f32x4 pe, ls;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int hd = 4 * g + i;
-      st_dev_f32(mlo + hd * 2, m[i]);
-      st_dev_f32(mlo + hd * 2 + 1, L.red[0][hd] + L.red[1][hd] + L.red[2][hd] + L.red[3][hd]);
+      for (int i = 0; i < 4; ++i) {
+        m[i] = fmaxf(fmaxf(rd[0][i], rd[1][i]), fmaxf(rd[2][i], rd[3][i]));
+        pe[i] = (valid && m[i] != -INFINITY) ? expf(sv[i] - m[i]) : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ls[i] = row16_sum(pe[i]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) L.p[(4 * g + i) * (MLA_SPLIT + 8) + key] = f32_to_bf16(pe[i] * ksk);
+      if (c16 == 0) *(f32x4*)&L.suml[wave][4 * g] = ls;
     }
-  }
-  // PV: wave w takes dim tiles TPW*w .. +TPW-1 (16 dims each), 2 key steps of 32
-  constexpr int TPW = 32 / NW;
-  bf16x8 pa[2];
+    __syncthreads();
+    if (have && wave == 0 && c16 == 0) {
+      const DevOut out(p.part_ml + ((size_t)r * p.nsplit + s) * MLA_HEADS * 2, MLA_HEADS * 8);
+      f32x4 l4 = *(const f32x4*)&L.suml[0][4 * g];
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks)
-    pa[ks] = __builtin_bit_cast(bf16x8, *(const uint4*)(L.p + c16 * (MLA_SPLIT + 8) + 32 * ks + 8 * g));
-  bf16_t* orow = p.part_o + ((size_t)r * p.nsplit + s) * MLA_HEADS * MLA_LAT;
-  static_assert(TPW % 2 == 0, "dim tiles go in pairs");
+      for (int w = 1; w < 4; ++w) l4 += *(const f32x4*)&L.suml[w][4 * g];
 #pragma unroll
-  for (int t = 0; t < TPW; t += 2) {
-    const int d0 = (wave * TPW + t) * 16;
-    f32x4 o[2];
+      for (int i = 0; i < 4; i += 2)
+        out.st16((4 * g + i) * 8, make_uint4(__float_as_uint(m[i]), __float_as_uint(l4[i]),
+                                                    __float_as_uint(m[i + 1]), __float_as_uint(l4[i + 1])));
+    }
+    // PV, the dims as the MFMA's rows and the heads as its columns: wave w takes dim tiles
+    // TPW*w .. +TPW-1 (16 dims each), 2 key steps of 32
+    constexpr int TPW = 32 / NW;
+    if (have) {
+      bf16x8 pa[2];
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-      o[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int ks = 0; ks < 2; ++ks)
+        pa[ks] = __builtin_bit_cast(bf16x8, *(const uint4*)(L.p + c16 * (MLA_SPLIT + 8) + 32 * ks + 8 * g));
+      const DevOut out(p.part_o + ((size_t)r * p.nsplit + s) * MLA_HEADS * MLA_LAT, MLA_HEADS * MLA_LAT * 2);
+      static_assert(TPW % 2 == 0, "dim tiles go in pairs");
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        const int w = (8 * ks + 2 * g) ^ mla_vswz(d0 + 16 * tt);  // d0 + c16 shares d0 >> 4
-        const uint2 vw = *(const uint2*)(L.vt + (d0 + 16 * tt + c16) * MLA_VROW + 4 * w);
-        o[tt] = mfma_bf16(pa[ks], e4m3x8_to_bf16(vw.x, vw.y), o[tt]);
+      for (int tl = 0; tl < TPW; tl += 2) {
+        const int d0 = (wave * TPW + tl) * 16;
+        uint32_t w[2][2];  // lane (c16, g): dims 4g .. 4g + 3 of head c16, two tiles, as bf16 pairs
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+          f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks) {
+            const uint2 vw = lds_read_keys8(L.k, 32 * ks + 8 * g, d0 + 16 * tt, c16);
+            o = mfma_bf16(e4m3x8_to_bf16(vw.x, vw.y), pa[ks], o);
+          }
+          w[tt][0] = pack_bf16x2(o[0], o[1]);
+          w[tt][1] = pack_bf16x2(o[2], o[3]);
+        }
+        // the second tile's even lane rows swapped with the first's odd ones: every lane then
+        // holds 8 consecutive dims (first tile: g 0, 2; second: g 1, 3), and a head's four
+        // lanes store one whole 64-byte piece
+        const auto lo = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+        out.st16((c16 * MLA_LAT + d0 + 16 * (g & 1) + 8 * (g >> 1)) * 2, make_uint4(lo[0], hi[0], lo[1], hi[1]));
       }
     }
-    // the pair's 32 columns as bf16 pairs, lane c16 taking columns 2 c16, 2 c16 + 1 of
-    // them (from lanes 2 c16 and 2 c16 + 1 of the first tile, or of the second), so
-    // that a row's 16 lanes store one whole 64-byte piece (half the bytes the merge
-    // tasks read, each (row, head) twice)
-    const int src = ((lane & 48) | ((2 * c16) & 15)) * 4;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int a0 = __builtin_amdgcn_ds_bpermute(src, __float_as_int(o[0][i]));
-      const int a1 = __builtin_amdgcn_ds_bpermute(src + 4, __float_as_int(o[0][i]));
-      const int b0 = __builtin_amdgcn_ds_bpermute(src, __float_as_int(o[1][i]));
-      const int b1 = __builtin_amdgcn_ds_bpermute(src + 4, __float_as_int(o[1][i]));
-      const bool first = c16 < 8;
-      st_dev_u32(orow + (4 * g + i) * MLA_LAT + d0 + 2 * c16,
-                 pack_bf16x2(__int_as_float(first ? a0 : b0), __int_as_float(first ? a1 : b1)));
-    }
+    if (HALF && i0 + 1 < iters) __syncthreads();  // the next task's rows replace these
   }
+  drain_memory();
   __syncthreads();
+  if (tid == 0 && any && t1 - t0 == iters) done(t1 - 1);
   return true;
 }
 

@@ -74,6 +74,33 @@ def test_mla_32_rows():
     assert e_lat <= REL_L2 and e_out <= REL_L2, (e_lat, e_out)
 
 
+@pytest.mark.parametrize("rows, topk", [(17, 64), (17, 512), (18, 2048), (27, 1984), (31, 4096)])
+def test_mla_above_16_rows_matches_narrow_calls(rows, topk):
+    """Above 16 rows the splits run two at a time, an equal run of them on each half
+    workgroup (none or one on most at the first shapes; runs that cross rows at the last
+    ones): the bits of the same rows in calls of at most 16, which run them one by one.
+    Some rows have unused slots, one row none in use."""
+    from sgl_amd_mono.k2 import config as C
+    from sgl_amd_mono.k2 import synth
+    from sgl_amd_mono.k2.ops import SparseMlaOp
+
+    dev = _dev()
+    cfg = C.MlaConfig(context=4096, topk=topk, hidden=1024)
+    ns = synth.make_mla(cfg, rows, rows + topk, dev)
+    ns.sel[1::3, topk // 3:] = -1
+    ns.sel[2, :] = -1
+    op = SparseMlaOp(cfg, ns, rows, ns.page_table.shape[1], device=dev)
+    args = (ns.kv, ns.kv_scale, ns.page_table)
+    for _ in range(2):  # the second launch on the workspace the first left
+        out = cpu(op(ns.q, *args, ns.req_ids, ns.sel, h=ns.h))
+        for a in range(0, rows, 9):
+            b = min(rows, a + 9)
+            part = SparseMlaOp(cfg, ns, b - a, ns.page_table.shape[1], device=dev)(
+                ns.q[a:b].contiguous(), *args, ns.req_ids[a:b].contiguous(), ns.sel[a:b].contiguous(), h=ns.h[a:b].contiguous())
+            assert torch.equal(cpu(part), out[a:b]), (a, b)
+    assert op.status() == 0
+
+
 def test_mla_unscaled_cache():
     """kv_scale None (SGLang's [slots][576] e4m3 cache) reads every row at scale 1:
     the oracle over unit scales, and bit-identical to passing a tensor of ones."""
