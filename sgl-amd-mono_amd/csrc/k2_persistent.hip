@@ -94,6 +94,19 @@ union K2Lds {
 };
 static_assert(sizeof(FrontLds) <= sizeof(TopkLds), "the front's LDS fits the layer's union as it is");
 
+// The launch's K2Dev (each kernel's first argument) as its kernel-argument memory, behind a
+// pointer the compiler cannot see through: a stage that takes it anew loads the pointers
+// and sizes it uses as it starts (scalar cache hits).  With one view of the arguments for
+// the whole walk they were loaded up front and lived, spilled to vector lanes, through
+// every stage: 205 of them at 32 rows and 264 at 8 of the A8W4 layer, now 96 and 116 (vector
+// spills at 32 rows 38 -> 24), and the layer 225.7 -> 214.4 us at 32 rows, the indexer's
+// launch 23.4 -> 22.9 at 8 x 65536.
+MK2_DEV const K2Dev* k2_args() {
+  auto a = (const __attribute__((address_space(4))) K2Dev*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return (const K2Dev*)a;
+}
+
 MK2_DEV int* k2_ctr(const K2Dev& p, int line) { return p.sync + line * SY_LINE; }
 
 // one finished task onto a counter, by a thread whose workgroup's stores have drained
@@ -288,26 +301,28 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
   // failure seen while polling) returns from the walk: the workgroup skips every task
   // left and goes straight to the counter reset (fail-stop)
   auto walk = [&]() {
+    const K2Dev* pp = k2_args();
     int base = 0;  // this stage's first workgroup
     // the tasks of a stage of n tasks on this workgroup; `t < G` marks the first
 #define K2_TASKS(t, n) for (int t = (b - base % G + G) % G; t < (n); t += G)
 #define K2_NEXT(n) base = (base + (n)) % G
     int st = 0;  // timeline stage
     // ---- index scores + row key histograms
-    k2_stamp(p, 3 * st);
-    const int nchk = p.idx.nchk;
+    k2_stamp(*pp, 3 * st);
+    const int nchk = pp->idx.nchk;
     auto keep_of = [&](int t) { return t / G < K2_KEEP ? kept[t / G] : nullptr; };
     K2_TASKS(t, R * nchk) {
-      idx_score<K2_NT>(p.idx, t / nchk, t % nchk, S.score, keep_of(t));
-      k2_signal(p, SY_SCORE + t / nchk);
+      idx_score<K2_NT>(pp->idx, t / nchk, t % nchk, S.score, keep_of(t));
+      k2_signal(*pp, SY_SCORE + t / nchk);
     }
-    k2_stamp(p, 3 * st++ + 2);
+    k2_stamp(*pp, 3 * st++ + 2);
     if (threadIdx.x == 0) s_tag = tag_of(epoch);
     __syncthreads();
     tp.tag = s_tag;
+    pp = k2_args();
     // ---- top-k slices: each chunk lists its keys above the row's threshold bin and
     // keeps its keys in the bin
-    k2_stamp(p, 3 * st);
+    k2_stamp(*pp, 3 * st);
     // slices on the workgroups of their score chunks (base unchanged).  A slice counts
     // out once its chunk's counts and bin keys are out.  With one slice a workgroup
     // (up to 8 rows) the last to count out of a row lists its own keys above the bin,
@@ -321,151 +336,158 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
     uint32_t sel_rows = 0;
     K2_TASKS(t, R * nchk) {
       const int r = t / nchk;
-      if (!k2_wait(p, seen, SY_SCORE + r, nchk, t < G ? 3 * st + 1 : -1)) return;
+      if (!k2_wait(*pp, seen, SY_SCORE + r, nchk, t < G ? 3 * st + 1 : -1)) return;
       bool last = false;
-      const bool known = idx_slice<K2_NT>(p.idx, r, t % nchk, S.topk, p.wait_ticks, k2_ctr(p, SY_ERR), tp.tag,
+      const bool known = idx_slice<K2_NT>(pp->idx, r, t % nchk, S.topk, pp->wait_ticks, k2_ctr(*pp, SY_ERR), tp.tag,
                                           [&] {
                                             if (sel_tasks)
-                                              k2_signal(p, SY_SLICE + r);
+                                              k2_signal(*pp, SY_SLICE + r);
                                             else
-                                              last = k2_signal_last1(p, SY_SLICE + r, nchk, &last_flag);
+                                              last = k2_signal_last1(*pp, SY_SLICE + r, nchk, &last_flag);
                                           },
                                           keep_of(t));
       if (last) {
-        k2_stamp(p, 3 * (st + 1));
-        k2_stamp(p, 3 * (st + 1) + 1);
+        k2_stamp(*pp, 3 * (st + 1));
+        k2_stamp(*pp, 3 * (st + 1) + 1);
         // this workgroup's own slice of row r may have left the threshold in LDS
-        idx_select<K2_NT>(p.idx, r, S.topk, tp.tag, known);
-        k2_stamp(p, 3 * (st + 1) + 2);
+        idx_select<K2_NT>(pp->idx, r, S.topk, tp.tag, known);
+        k2_stamp(*pp, 3 * (st + 1) + 2);
         sel_rows |= 1u << r;
       }
     }
-    k2_stamp(p, 3 * st + 2);
+    k2_stamp(*pp, 3 * st + 2);
     K2_NEXT(R * nchk);
     if (sel_tasks) {
       K2_TASKS(r, R) {
-        k2_stamp(p, 3 * (st + 1));
-        if (!k2_wait(p, seen, SY_SLICE + r, nchk, 3 * (st + 1) + 1)) return;
-        idx_select<K2_NT>(p.idx, r, S.topk, tp.tag, false);
-        k2_stamp(p, 3 * (st + 1) + 2);
+        k2_stamp(*pp, 3 * (st + 1));
+        if (!k2_wait(*pp, seen, SY_SLICE + r, nchk, 3 * (st + 1) + 1)) return;
+        idx_select<K2_NT>(pp->idx, r, S.topk, tp.tag, false);
+        k2_stamp(*pp, 3 * (st + 1) + 2);
         sel_rows |= 1u << r;
       }
       K2_NEXT(R);
     }
     st += 2;  // the select stamps are taken above
+    pp = k2_args();
     // ---- sparse-MLA splits
-    k2_stamp(p, 3 * st);
-    const int ns = p.mla.nsplit;
+    k2_stamp(*pp, 3 * st);
+    const int ns = pp->mla.nsplit;
     // a split polls its 64 entries of the tagged list: it starts as soon as they are out
     // (most come from the slices, ahead of the row's select)
-    if (!k2_splits<NCG>(p, S, (b - base % G + G) % G, tp, [&](int) { k2_stamp(p, 3 * st + 1); })) return;
+    if (!k2_splits<NCG>(*pp, S, (b - base % G + G) % G, tp, [&](int) { k2_stamp(*pp, 3 * st + 1); })) return;
     K2_NEXT(R * ns);
-    k2_stamp(p, 3 * st++ + 2);
+    k2_stamp(*pp, 3 * st++ + 2);
+    pp = k2_args();
     // ---- merge of the splits + W_UV, per (group of mrg rows, head, half of the head's
     // outputs): about one task a workgroup
-    k2_stamp(p, 3 * st);
+    k2_stamp(*pp, 3 * st);
     const int mrg = mla_merge_rows(R, G), nmt = 2 * MLA_HEADS * ((R + mrg - 1) / mrg);
     K2_TASKS(t, nmt) {
       const int r0 = t / (2 * MLA_HEADS) * mrg, nr = min(mrg, R - r0), h = (t >> 1) % MLA_HEADS;
-      mla_merge_uv<K2_NT>(p.mla, r0, nr, h, t & 1, S.merge, [&] {
+      mla_merge_uv<K2_NT>(pp->mla, r0, nr, h, t & 1, S.merge, [&] {
         for (int i = 0; i < nr; ++i)
-          if (!k2_wait(p, seen, SY_SPLIT + r0 + i, ns, t < G && i == nr - 1 ? 3 * st + 1 : -1)) return false;
+          if (!k2_wait(*pp, seen, SY_SPLIT + r0 + i, ns, t < G && i == nr - 1 ? 3 * st + 1 : -1)) return false;
         return true;
       });
       if (seen[SY_LINES]) return;
-      k2_signal(p, SY_UV, t, K2_LANES);
+      k2_signal(*pp, SY_UV, t, K2_LANES);
     }
     K2_NEXT(nmt);
-    k2_stamp(p, 3 * st++ + 2);
+    k2_stamp(*pp, 3 * st++ + 2);
+    pp = k2_args();
     // ---- W_o + residual, per 16 hidden rows: tasks t and t + G together (their weights
     // all in flight before the wait)
-    k2_stamp(p, 3 * st);
-    const int ht = p.mla.hidden / 16;
+    k2_stamp(*pp, 3 * st);
+    const int ht = pp->mla.hidden / 16;
     for (int t = (b - base % G + G) % G; t < ht; t += 2 * G) {
       const int t1 = t + G < ht ? t + G : -1;
-      mla_oproj<K2_NT, NCG, 2>(p.mla, t, t1, S.up.red,
-                               [&] { return k2_wait(p, seen, SY_UV, nmt, t < G ? 3 * st + 1 : -1, K2_LANES); });
+      mla_oproj<K2_NT, NCG, 2>(pp->mla, t, t1, S.up.red,
+                               [&] { return k2_wait(*pp, seen, SY_UV, nmt, t < G ? 3 * st + 1 : -1, K2_LANES); });
       if (seen[SY_LINES]) return;
-      k2_signal(p, SY_OPROJ, t, K2_LANES, t1 >= 0 ? 2 : 1);
+      k2_signal(*pp, SY_OPROJ, t, K2_LANES, t1 >= 0 ? 2 : 1);
     }
     K2_NEXT(ht);
-    k2_stamp(p, 3 * st++ + 2);
+    k2_stamp(*pp, 3 * st++ + 2);
+    pp = k2_args();
     // ---- router GEMV (+ RMSNorm of its slice), per (16 experts, hidden slice): the
     // partial logits go out as tagged words (the routing polls them); the counter
     // publishes the normalized rows the tasks of the first expert tile store
-    k2_stamp(p, 3 * st);
-    const int et = p.moe.E / 16, nrt = et * p.moe.KC;
+    k2_stamp(*pp, 3 * st);
+    const int et = pp->moe.E / 16, nrt = et * pp->moe.KC;
     K2_TASKS(t, nrt) {
-      moe_router<K2_NT, NCG, FMT>(p.moe, t % et, t / et, S.router, tp.tag,
-                             [&] { return k2_wait(p, seen, SY_OPROJ, ht, t < G ? 3 * st + 1 : -1, K2_LANES); });
+      moe_router<K2_NT, NCG, FMT>(pp->moe, t % et, t / et, S.router, tp.tag,
+                             [&] { return k2_wait(*pp, seen, SY_OPROJ, ht, t < G ? 3 * st + 1 : -1, K2_LANES); });
       if (seen[SY_LINES]) return;
-      k2_signal(p, SY_ROUTER, t, K2_LANES);
+      k2_signal(*pp, SY_ROUTER, t, K2_LANES);
     }
     K2_NEXT(nrt);
-    k2_stamp(p, 3 * st++ + 2);
+    k2_stamp(*pp, 3 * st++ + 2);
+    pp = k2_args();
     // ---- routing, on one workgroup up to 8 rows: one without a router task (it polls
     // while they run) and with the fewest up/gate tasks.  It polls the router tasks' logits and
     // puts out the tagged expert list, then the route-weight table, published by
     // SY_ROUTE for the down
-    const int up_r = p.moe.Dmax * (p.moe.I / p.moe.UC);
-    const int up_sh = p.moe.n_shared * (p.moe.SI / 32);
+    const int up_r = pp->moe.Dmax * (pp->moe.I / pp->moe.UC);
+    const int up_sh = pp->moe.n_shared * (pp->moe.SI / 32);
     const int up_total = up_r + up_sh;
     // the up/gate tasks start at workgroup `base`; from base + up_total % G on, the
     // workgroups hold one fewer; the router tasks ended on the nrt workgroups before base
     // above 8 rows the rows' top-k runs on nq workgroups of 8 rows each, the first of
     // which (the lead) polls the others' picks and puts out the list and the tables
-    const int nq = p.moe.M > 8 ? (p.moe.M + 7) / 8 : 1;
+    const int nq = pp->moe.M > 8 ? (pp->moe.M + 7) / 8 : 1;
     int route_at = up_total % G;
     if (nrt < G && route_at > G - nrt - nq) route_at = max(0, G - nrt - nq);
     const int q = (b - base - route_at + 2 * G) % G;
     if (q < nq) {
       constexpr bool CMP = kCompact<NCG, FMT>;
-      if (q == 0) k2_stamp(p, 3 * st);
-      auto mark = [&](int i) { if (q == 0) k2_stamp(p, 3 * K2_STAGES + i); };
+      if (q == 0) k2_stamp(*pp, 3 * st);
+      auto mark = [&](int i) { if (q == 0) k2_stamp(*pp, 3 * K2_STAGES + i); };
       bool ok;
       if (nq == 1)
-        ok = moe_route<K2_NT, CMP>(p.moe, S.route, tp, mark);
+        ok = moe_route<K2_NT, CMP>(pp->moe, S.route, tp, mark);
       else if (q == 0)
-        ok = moe_route<K2_NT, CMP, ROUTE_LEAD>(p.moe, S.route, tp, mark, 0, 8);
+        ok = moe_route<K2_NT, CMP, ROUTE_LEAD>(pp->moe, S.route, tp, mark, 0, 8);
       else
-        ok = moe_route<K2_NT, CMP, ROUTE_PICK>(p.moe, S.route, tp, mark, 8 * q, min(p.moe.M, 8 * q + 8));
+        ok = moe_route<K2_NT, CMP, ROUTE_PICK>(pp->moe, S.route, tp, mark, 8 * q, min(pp->moe.M, 8 * q + 8));
       if (!ok) return;
       if (q == 0) {
-        k2_stamp(p, 3 * st + 1);
-        k2_signal(p, SY_ROUTE);
-        k2_stamp(p, 3 * st + 2);
+        k2_stamp(*pp, 3 * st + 1);
+        k2_signal(*pp, SY_ROUTE);
+        k2_stamp(*pp, 3 * st + 2);
       }
     }
     ++st;
+    pp = k2_args();
     // ---- up/gate + SwiGLU: the shared expert's chunks first (they need only the
     // normalized rows, so they run while routing is still pending), then the routed
     // slots, each polling its slot of the tagged expert list
-    k2_stamp(p, 3 * st);
+    k2_stamp(*pp, 3 * st);
     // the selects' rows' histograms back to zero, here where a workgroup waits for the
     // routing anyway (every slice and select read them long ago; a stopped launch
     // leaves this to the last workgroup out)
-    for (uint32_t m = sel_rows; m; m &= m - 1) idx_clear_hist<K2_NT>(p.idx, __ffs((int)m) - 1);
+    for (uint32_t m = sel_rows; m; m &= m - 1) idx_clear_hist<K2_NT>(pp->idx, __ffs((int)m) - 1);
     if constexpr (NCG == 1) {
       K2_TASKS(t, up_total) {
         const bool sh = t < up_sh;
-        if (!k2_wait(p, seen, SY_ROUTER, nrt, t < G ? 3 * st + 1 : -1, K2_LANES)) return;
-        if (moe_upgate<K2_NT, NCG, FMT>(p.moe, sh ? up_r + t : t - up_sh, S.up.red, S.up.midf, tp) < 0) return;
-        k2_signal(p, SY_UP, t, K2_LANES);
+        if (!k2_wait(*pp, seen, SY_ROUTER, nrt, t < G ? 3 * st + 1 : -1, K2_LANES)) return;
+        if (moe_upgate<K2_NT, NCG, FMT>(pp->moe, sh ? up_r + t : t - up_sh, S.up.red, S.up.midf, tp) < 0) return;
+        k2_signal(*pp, SY_UP, t, K2_LANES);
       }
-    } else if (!k2_upgate_walk<NCG, FMT>(p, S, seen, &up_next, (b - base % G + G) % G, nrt, tp, 3 * st + 1)) {
+    } else if (!k2_upgate_walk<NCG, FMT>(*pp, S, seen, &up_next, (b - base % G + G) % G, nrt, tp, 3 * st + 1)) {
       return;
     }
     K2_NEXT(up_total);
-    k2_stamp(p, 3 * st++ + 2);
+    k2_stamp(*pp, 3 * st++ + 2);
+    pp = k2_args();
     // ---- down + route weighting + residual, per 16 hidden rows
-    k2_stamp(p, 3 * st);
-    K2_TASKS(t, down_tasks(p.moe)) {
-      if (!k2_wait(p, seen, SY_ROUTE, 1)) return;  // the routing and its table: known long before the mid rows
-      moe_down<K2_NT, NCG, FMT>(p.moe, t, S.down.red, S.down.act, S.down.xres,
-                                [&] { return k2_upgate_done<NCG>(p, seen, t < G ? 3 * st + 1 : -1); });
+    k2_stamp(*pp, 3 * st);
+    K2_TASKS(t, down_tasks(pp->moe)) {
+      if (!k2_wait(*pp, seen, SY_ROUTE, 1)) return;  // the routing and its table: known long before the mid rows
+      moe_down<K2_NT, NCG, FMT>(pp->moe, t, S.down.red, S.down.act, S.down.xres,
+                                [&] { return k2_upgate_done<NCG>(*pp, seen, t < G ? 3 * st + 1 : -1); });
       if (seen[SY_LINES]) return;
     }
-    k2_stamp(p, 3 * st + 2);
+    k2_stamp(*pp, 3 * st + 2);
 
   };
   // the front first, when the launch runs it: a failed front stops the layer's walk and
@@ -593,68 +615,76 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_block(K2Dev p) {
   const TagPoll tp{s_tag, p.wait_ticks, k2_ctr(p, SY_ERR)};
   uint32_t sel_rows = 0;  // the rows whose select this workgroup ran
   auto walk = [&]() {
+    // a new view a stage; one for the whole walk in the W8A8 MoE block, which ran 4 % slower
+    // with one a stage (117.5 -> 122.3 us at 13 rows)
+    constexpr bool one_view = BLK == K2_BLOCK_MOE && FMT == MK2_FMT_W8A8;
+    const K2Dev* pp = one_view ? &p : k2_args();
+    auto next_view = [&] { if (!one_view) pp = k2_args(); };
     int base = 0;
 #define K2_TASKS(t, n) for (int t = (b - base % G + G) % G; t < (n); t += G)
 #define K2_NEXT(n) base = (base + (n)) % G
     if constexpr (BLK == K2_BLOCK_INDEXER) {
       // scores, slices (the last of a row to count out runs its select with one slice a
       // workgroup; with several, the selects are tasks of their own): as the layer's
-      const int nchk = p.idx.nchk;
+      const int nchk = pp->idx.nchk;
       auto keep_of = [&](int t) { return t / G < K2_KEEP ? kept[t / G] : nullptr; };
       K2_TASKS(t, R * nchk) {
-        idx_score<K2_NT>(p.idx, t / nchk, t % nchk, S.score, keep_of(t));
-        k2_signal(p, SY_SCORE + t / nchk);
+        idx_score<K2_NT>(pp->idx, t / nchk, t % nchk, S.score, keep_of(t));
+        k2_signal(*pp, SY_SCORE + t / nchk);
       }
+      next_view();
       const bool sel_tasks = R * nchk > G;
       K2_TASKS(t, R * nchk) {
         const int r = t / nchk;
-        if (!k2_wait(p, seen, SY_SCORE + r, nchk)) return;
+        if (!k2_wait(*pp, seen, SY_SCORE + r, nchk)) return;
         bool last = false;
-        const bool known = idx_slice<K2_NT>(p.idx, r, t % nchk, S.topk, p.wait_ticks, k2_ctr(p, SY_ERR), tp.tag,
+        const bool known = idx_slice<K2_NT>(pp->idx, r, t % nchk, S.topk, pp->wait_ticks, k2_ctr(*pp, SY_ERR), tp.tag,
                                             [&] {
                                               if (sel_tasks)
-                                                k2_signal(p, SY_SLICE + r);
+                                                k2_signal(*pp, SY_SLICE + r);
                                               else
-                                                last = k2_signal_last1(p, SY_SLICE + r, nchk, &last_flag);
+                                                last = k2_signal_last1(*pp, SY_SLICE + r, nchk, &last_flag);
                                             },
                                             keep_of(t));
         if (last) {
-          idx_select<K2_NT>(p.idx, r, S.topk, tp.tag, known);
+          idx_select<K2_NT>(pp->idx, r, S.topk, tp.tag, known);
           sel_rows |= 1u << r;
         }
       }
       K2_NEXT(R * nchk);
       if (sel_tasks) {
         K2_TASKS(r, R) {
-          if (!k2_wait(p, seen, SY_SLICE + r, nchk)) return;
-          idx_select<K2_NT>(p.idx, r, S.topk, tp.tag, false);
+          if (!k2_wait(*pp, seen, SY_SLICE + r, nchk)) return;
+          idx_select<K2_NT>(pp->idx, r, S.topk, tp.tag, false);
           sel_rows |= 1u << r;
         }
       }
       // every slice and select read the histograms: the selects' rows back to zero
-      for (uint32_t m = sel_rows; m; m &= m - 1) idx_clear_hist<K2_NT>(p.idx, __ffs((int)m) - 1);
+      for (uint32_t m = sel_rows; m; m &= m - 1) idx_clear_hist<K2_NT>(pp->idx, __ffs((int)m) - 1);
     } else if constexpr (BLK == K2_BLOCK_MLA) {
       // splits (the given positions), merge + W_UV, W_o + residual: as the layer's
-      const int ns = p.mla.nsplit;
-      if (!k2_splits<NCG>(p, S, b, tp)) return;
+      const int ns = pp->mla.nsplit;
+      if (!k2_splits<NCG>(*pp, S, b, tp)) return;
       K2_NEXT(R * ns);
+      next_view();
       const int mrg = mla_merge_rows(R, G), nmt = 2 * MLA_HEADS * ((R + mrg - 1) / mrg);
       K2_TASKS(t, nmt) {
         const int r0 = t / (2 * MLA_HEADS) * mrg, nr = min(mrg, R - r0), h = (t >> 1) % MLA_HEADS;
-        mla_merge_uv<K2_NT>(p.mla, r0, nr, h, t & 1, S.merge, [&] {
+        mla_merge_uv<K2_NT>(pp->mla, r0, nr, h, t & 1, S.merge, [&] {
           for (int i = 0; i < nr; ++i)
-            if (!k2_wait(p, seen, SY_SPLIT + r0 + i, ns)) return false;
+            if (!k2_wait(*pp, seen, SY_SPLIT + r0 + i, ns)) return false;
           return true;
         });
         if (seen[SY_LINES]) return;
-        k2_signal(p, SY_UV, t, K2_LANES);
+        k2_signal(*pp, SY_UV, t, K2_LANES);
       }
       K2_NEXT(nmt);
-      const int ht = p.mla.hidden / 16;
+      next_view();
+      const int ht = pp->mla.hidden / 16;
       for (int t = (b - base % G + G) % G; t < ht; t += 2 * G) {
         const int t1 = t + G < ht ? t + G : -1;
-        mla_oproj<K2_NT, NCG, 2>(p.mla, t, t1, S.up.red,
-                                 [&] { return k2_wait(p, seen, SY_UV, nmt, -1, K2_LANES); });
+        mla_oproj<K2_NT, NCG, 2>(pp->mla, t, t1, S.up.red,
+                                 [&] { return k2_wait(*pp, seen, SY_UV, nmt, -1, K2_LANES); });
         if (seen[SY_LINES]) return;
       }
     } else {
@@ -662,24 +692,26 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_block(K2Dev p) {
       // as the layer's, the sums from tasks of their own (the layer's come from W_o)
       // (512 columns a task on the first 128 threads: the staged kernel's shape, so both
       // give the same bits for any hidden size a multiple of 512)
-      const int per = p.moe.H / 512, nss = p.moe.norm ? p.rows * per : 0;
+      const int per = pp->moe.H / 512, nss = pp->moe.norm ? pp->rows * per : 0;
       K2_TASKS(t, nss) {
-        if (threadIdx.x < 128) moe_sumsq<128>(p.moe, t / per, t % per);
-        k2_signal(p, SY_OPROJ, t, K2_LANES);
+        if (threadIdx.x < 128) moe_sumsq<128>(pp->moe, t / per, t % per);
+        k2_signal(*pp, SY_OPROJ, t, K2_LANES);
       }
       K2_NEXT(nss);
-      const int et = p.moe.E / 16, nrt = et * p.moe.KC;
+      next_view();
+      const int et = pp->moe.E / 16, nrt = et * pp->moe.KC;
       K2_TASKS(t, nrt) {
-        moe_router<K2_NT, NCG, FMT>(p.moe, t % et, t / et, S.router, tp.tag,
-                                    [&] { return k2_wait(p, seen, SY_OPROJ, nss, -1, K2_LANES); });
+        moe_router<K2_NT, NCG, FMT>(pp->moe, t % et, t / et, S.router, tp.tag,
+                                    [&] { return k2_wait(*pp, seen, SY_OPROJ, nss, -1, K2_LANES); });
         if (seen[SY_LINES]) return;
-        k2_signal(p, SY_ROUTER, t, K2_LANES);
+        k2_signal(*pp, SY_ROUTER, t, K2_LANES);
       }
       K2_NEXT(nrt);
-      const int up_r = p.moe.Dmax * (p.moe.I / p.moe.UC);
-      const int up_sh = p.moe.n_shared * (p.moe.SI / 32);
+      const int up_r = pp->moe.Dmax * (pp->moe.I / pp->moe.UC);
+      const int up_sh = pp->moe.n_shared * (pp->moe.SI / 32);
       const int up_total = up_r + up_sh;
-      const int nq = p.moe.M > 8 ? (p.moe.M + 7) / 8 : 1;
+      next_view();
+      const int nq = pp->moe.M > 8 ? (pp->moe.M + 7) / 8 : 1;
       int route_at = up_total % G;
       if (nrt < G && route_at > G - nrt - nq) route_at = max(0, G - nrt - nq);
       const int q = (b - base - route_at + 2 * G) % G;
@@ -687,20 +719,22 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_block(K2Dev p) {
         constexpr bool CMP = kCompact<NCG, FMT>;
         bool ok;
         if (nq == 1)
-          ok = moe_route<K2_NT, CMP>(p.moe, S.route, tp);
+          ok = moe_route<K2_NT, CMP>(pp->moe, S.route, tp);
         else if (q == 0)
-          ok = moe_route<K2_NT, CMP, ROUTE_LEAD>(p.moe, S.route, tp, NoMark(), 0, 8);
+          ok = moe_route<K2_NT, CMP, ROUTE_LEAD>(pp->moe, S.route, tp, NoMark(), 0, 8);
         else
-          ok = moe_route<K2_NT, CMP, ROUTE_PICK>(p.moe, S.route, tp, NoMark(), 8 * q, min(p.moe.M, 8 * q + 8));
+          ok = moe_route<K2_NT, CMP, ROUTE_PICK>(pp->moe, S.route, tp, NoMark(), 8 * q, min(pp->moe.M, 8 * q + 8));
         if (!ok) return;
-        if (q == 0) k2_signal(p, SY_ROUTE);
+        if (q == 0) k2_signal(*pp, SY_ROUTE);
       }
-      if (!k2_upgate_walk<NCG, FMT>(p, S, seen, &up_next, (b - base % G + G) % G, nrt, tp, -1)) return;
+      next_view();
+      if (!k2_upgate_walk<NCG, FMT>(*pp, S, seen, &up_next, (b - base % G + G) % G, nrt, tp, -1)) return;
       K2_NEXT(up_total);
-      K2_TASKS(t, down_tasks(p.moe)) {
-        if (!k2_wait(p, seen, SY_ROUTE, 1)) return;
-        moe_down<K2_NT, NCG, FMT>(p.moe, t, S.down.red, S.down.act, S.down.xres,
-                                  [&] { return k2_upgate_done<NCG>(p, seen, -1); });
+      next_view();
+      K2_TASKS(t, down_tasks(pp->moe)) {
+        if (!k2_wait(*pp, seen, SY_ROUTE, 1)) return;
+        moe_down<K2_NT, NCG, FMT>(pp->moe, t, S.down.red, S.down.act, S.down.xres,
+                                  [&] { return k2_upgate_done<NCG>(*pp, seen, -1); });
         if (seen[SY_LINES]) return;
       }
     }
