@@ -85,11 +85,7 @@ size_t moe_carve(const mk2_moe_shape* s, void* base, MoeDev* d) {
   // up/gate chunks: 128 intermediate rows for W8A8 (its mid is quantized per 128), 64
   // for E2M1 weights up to 16 rows, else 32
   t.UC = fmt == MK2_FMT_W8A8 ? 128 : (w_fp4(fmt) && M <= 16 && I % 64 == 0) ? 64 : 32;
-  // down tasks: 24 hidden rows when hidden is a multiple of 48 (6144: one task a CU of
-  // MI355X), for the scaled-MFMA E2M1 modes (above 16 rows on compacted rows); else 32
-  // for them up to 16 rows; 16 otherwise
-  const bool mx_down = fmt == MK2_FMT_MXFP4 || fmt == MK2_FMT_A4W4;
-  t.DT = !mx_down ? 1 : H % 48 == 0 ? 3 : (M <= 16 && H % 32 == 0) ? 2 : 1;
+  t.DR = down_task_rows(H);
   t.ssp = c.take<float>((size_t)(H / 16) * M);
   t.xn = c.take<bf16_t>((size_t)M * H);
   t.xq = c.take<uint8_t>((size_t)M * H);
@@ -113,7 +109,7 @@ size_t moe_carve(const mk2_moe_shape* s, void* base, MoeDev* d) {
   }
   t.mid_sh = c.take<bf16_t>((size_t)M * (s->n_shared ? s->shared_inter : 0) + 1);
   if (d) {
-    d->KC = t.KC; d->Dmax = t.Dmax; d->UC = t.UC; d->DT = t.DT; d->ssp = t.ssp; d->xn = t.xn; d->xq = t.xq; d->xs = t.xs;
+    d->KC = t.KC; d->Dmax = t.Dmax; d->UC = t.UC; d->DR = t.DR; d->ssp = t.ssp; d->xn = t.xn; d->xq = t.xq; d->xs = t.xs;
     d->xsf = t.xsf; d->mid_sf = t.mid_sf;
     d->logit_part = t.logit_part; d->logits = t.logits; d->topk_ids = t.topk_ids;
     d->topk_w = t.topk_w; d->act = t.act; d->rw = t.rw; d->mid_q = t.mid_q;

@@ -23,8 +23,7 @@ struct MoeDev {
   int KC;    // router k-chunks
   int Dmax;  // capacity of the distinct-expert list
   int UC;    // intermediate rows of a routed up/gate task (64: MXFP4 at <= 16 rows, else 32)
-  int DT;    // 16-row hidden tiles of a down task (2: MXFP4 at <= 16 rows, else 1; 3: 24 rows,
-            // a tile and a half, when hidden is a multiple of 48)
+  int DR;    // hidden rows of a down task: 16, 24 or 32 (down_task_rows)
   float route_scale, eps;
   int wl;    // MK2_WLAYOUT_*: the expert weights' layout
   const bf16_t* x;
@@ -1030,34 +1029,24 @@ MK2_DEV int moe_upgate(const MoeDev& p, int t, float* red, float* midf, const Ta
 }
 
 // ---------------------------------------------------------- stage: down + combine
-// A down task's hidden rows: tile tl[d], rows rlo[d] .. rhi[d] - 1 of it (every row of
-// DT tiles, or with p.DT == 3 (DT 2) 24 rows: a whole tile and half of the next, in
-// either order); c0 the first (its output column), ncol how many, live[d] whether
-// lane row c16 is one of tile d's
+// A down task's hidden rows: tile tl[d], rows rlo[d] .. rhi[d] - 1 of it (with DT 1 a whole
+// tile; with DT 2 two tiles, or p.DR == 24 a whole one and half of the next, in either
+// order); c0 the first (its output column), ncol how many, live[d] whether lane row c16 is
+// one of tile d's
 template <int DT>
 struct DownRows {
   int tl[DT], rlo[DT], rhi[DT], c0, ncol;
   bool live[DT];
   MK2_DEV DownRows(const MoeDev& p, int nt, int c16) {
+    c0 = DT == 1 ? nt * 16 : nt * p.DR;
+    ncol = DT == 1 ? 16 : p.DR;
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
-      tl[d] = nt * DT + d;
-      rlo[d] = 0;
-      rhi[d] = 16;
+      tl[d] = c0 / 16 + d;
+      rlo[d] = DT == 1 ? 0 : max(c0 - tl[d] * 16, 0);
+      rhi[d] = DT == 1 ? 16 : min(c0 + ncol - tl[d] * 16, 16);
+      live[d] = c16 >= rlo[d] && c16 < rhi[d];
     }
-    if (DT == 2 && p.DT == 3) {
-      const int ta = (3 * nt) >> 1;
-      tl[0] = ta;
-      tl[DT - 1] = ta + 1;
-      rlo[0] = nt & 1 ? 8 : 0;
-      rhi[DT - 1] = nt & 1 ? 16 : 8;
-    }
-    c0 = tl[0] * 16 + rlo[0];
-    ncol = 0;
-#pragma unroll
-    for (int d = 0; d < DT; ++d) ncol += rhi[d] - rlo[d];
-#pragma unroll
-    for (int d = 0; d < DT; ++d) live[d] = c16 >= rlo[d] && c16 < rhi[d];
   }
 };
 
@@ -1157,7 +1146,7 @@ MK2_DEV void down_epilogue(const MoeDev& p, const DownRows<DT>& t, float* red, c
   __syncthreads();
 }
 
-// A task is 16*DT hidden rows (24 with p.DT == 3); every slot (the shared expert, then the D routed
+// A task is p.DR hidden rows; every slot (the shared expert, then the D routed
 // experts) adds rw * W_down[e] . mid into the rows' accumulators; out = bf16(y [+ x]).
 // Waves take every NW-th slot, B slots a unit, the next unit's weight tiles and mid
 // rows (shared by the DT tiles) in flight while a unit's MFMAs run.  act_ids: LDS >=
@@ -1282,12 +1271,123 @@ MK2_DEV void down_rows(const MoeDev& p, int nt, float* red, int* act_ids, float*
       }
     }
   };
+  // the other modes' units, the same slots and passes one slot at a time: E4M3 weights (f32
+  // scale per 128 x 128 block) widened to bf16 against the bf16 mid (W8A16), or on the
+  // scaled MFMA against the E4M3 mid (W8A8, f32 scale per 128 a row), each k-block's product
+  // times its scales and the route weight; or E2M1 weights widened exactly to bf16 against
+  // the bf16 mid (A16W4), the slot's sum times the route weight.  DEPTH - 1 units are in
+  // flight while one computes, as many as the registers hold without spills.  Slot by slot
+  // (a slot's loads, then its products, in 16-row tasks) the block took 88.7 us at 8 rows of
+  // hidden 6144 (256 experts of 256) in W8A16 and 67 in A16W4, now 71.1 and 47.8; W8A8 at 13
+  // rows 117.6 -> 96.8
+  constexpr bool w8a8 = FMT == MK2_FMT_W8A8, a16w4 = FMT == MK2_FMT_A16W4;
+  constexpr int KCB = NCG == 1 || (w8a8 && DT == 1) ? 2 : 1;  // k-blocks a unit
+  constexpr int DEPTH = w8a8 ? (DT == 1 && NCG == 1 ? 3 : 2) : NCG == 2 || a16w4 ? 3 : 2;
+  struct UnitB {
+    uint4 a[DT][KCB][a16w4 ? 1 : 2];
+    i32x8 bq[w8a8 ? KCB : 1][NCG];        // W8A8
+    bf16x8 bb[w8a8 ? 1 : KCB][NCG][4];    // W8A16, A16W4
+    float sc[DT][KCB];                    // E4M3: the block scales
+    uint32_t sw[DT];                     // E2M1: the E8M0 words
+    float ms[w8a8 ? KCB : 1][NCG], wr[NCG];
+  };
+  const int nkcb = (KB2 + KCB - 1) / KCB;  // units a slot
+  const int nub = !mx && D > wave ? (D - wave + NW - 1) / NW * nkcb : 0;
+  auto load_wb = [&](int u, UnitB& x) {
+    const int e = act_ids[wave + (u / nkcb) * NW], kb0 = (u % nkcb) * KCB;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+#pragma unroll
+      for (int c = 0; c < KCB; ++c) {
+        const size_t blk = ((size_t)e * HT + tl[d]) * KB2 + min(kb0 + c, KB2 - 1);
+        const uint4 z = make_uint4(0, 0, 0, 0);
+        if constexpr (a16w4) {
+          x.a[d][c][0] = live[d] ? ld_stream16(p.w2 + blk * 1024 + lane * 16) : z;
+        } else {
+          x.a[d][c][0] = x.a[d][c][a16w4 ? 0 : 1] = z;
+          if (live[d]) load_fp8_block(p.w2 + blk * 2048, p.wl, lane, x.a[d][c][0], x.a[d][c][a16w4 ? 0 : 1]);
+          x.sc[d][c] = ((const float*)p.s2)[((size_t)e * (p.H / 128) + tl[d] / 8) * KB2 + min(kb0 + c, KB2 - 1)];
+        }
+      }
+      if constexpr (a16w4) x.sw[d] = e8m0_word(p.s2 + e * e8m0_expert_bytes(p.wl, p.H, p.I), p.wl, p.I, tl[d], kb0, lane);
+    }
+  };
+  auto load_mb = [&](int u, UnitB& x) {
+    const int j = wave + (u / nkcb) * NW, kb0 = (u % nkcb) * KCB;
+#pragma unroll
+    for (int cg = 0; cg < NCG; ++cg) {
+      const int row = cg * 16 + c16;
+#pragma unroll
+      for (int c = 0; c < KCB; ++c) {
+        const int kb = min(kb0 + c, KB2 - 1);
+        if constexpr (w8a8) {
+          x.bq[c][cg] = load_b_fp8_same(p.mid_q + (size_t)j * p.M * p.I, row, p.M, p.I, kb * 128, g);
+          x.ms[c][cg] = row < p.M ? ldp_f32(p.mid_sf + ((size_t)j * p.M + row) * (p.I / 128) + kb) : 0.f;
+        } else {
+          load_b_bf16(p.mid_b + (size_t)j * p.M * p.I, row, p.M, p.I, kb * 128 + 32 * g, x.bb[c][cg]);
+        }
+      }
+      x.wr[cg] = ldp_f32(p.rw + j * 32 + row);
+    }
+  };
+  f32x4 tb[DT][NCG];  // A16W4: the slot's sums
+  auto compute_b = [&](int u, UnitB& x) {
+    const int kb0 = (u % nkcb) * KCB;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      if (a16w4 && kb0 == 0) {
+#pragma unroll
+        for (int cg = 0; cg < NCG; ++cg) tb[d][cg] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int c = 0; c < KCB; ++c) {
+        if (kb0 + c >= KB2) break;
+        if constexpr (w8a8) {
+          const uint4 lo = x.a[d][c][0], hi = x.a[d][c][a16w4 ? 0 : 1];
+          const i32x8 A = {(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+#pragma unroll
+          for (int cg = 0; cg < NCG; ++cg)
+            acc[d][cg] += mfma_same<0>(A, x.bq[c][cg], f32x4{0.f, 0.f, 0.f, 0.f}, E8M0_ONE, E8M0_ONE) *
+                          (x.sc[d][c] * x.ms[c][cg] * x.wr[cg]);
+        } else if constexpr (a16w4) {
+          const float sc = e8m0_to_f32(x.sw[d] >> e8m0_shift(p.wl, tl[d], kb0 + c));
+          const uint4 w = x.a[d][c][0];
+          const bf16x8 a[4] = {e2m1x8_to_bf16(w.x, sc), e2m1x8_to_bf16(w.y, sc), e2m1x8_to_bf16(w.z, sc),
+                               e2m1x8_to_bf16(w.w, sc)};
+#pragma unroll
+          for (int cg = 0; cg < NCG; ++cg) tb[d][cg] = mfma4_bf16(a, x.bb[c][cg], tb[d][cg]);
+        } else {
+          const uint4 lo = x.a[d][c][0], hi = x.a[d][c][a16w4 ? 0 : 1];
+          const bf16x8 a[4] = {e4m3x8_to_bf16(lo.x, lo.y), e4m3x8_to_bf16(lo.z, lo.w), e4m3x8_to_bf16(hi.x, hi.y),
+                               e4m3x8_to_bf16(hi.z, hi.w)};
+#pragma unroll
+          for (int cg = 0; cg < NCG; ++cg)
+            acc[d][cg] += mfma4_bf16(a, x.bb[c][cg], f32x4{0.f, 0.f, 0.f, 0.f}) * (x.sc[d][c] * x.wr[cg]);
+        }
+      }
+      if (a16w4 && kb0 + KCB >= KB2) {
+#pragma unroll
+        for (int cg = 0; cg < NCG; ++cg) acc[d][cg] += tb[d][cg] * x.wr[cg];
+      }
+    }
+  };
   Unit x0, x1, x2;
-  if (nu > 0) load_w(0, x0);
-  if (nu > 1) load_w(1, x1);
+  UnitB y0, y1, y2;
+  if constexpr (mx) {
+    if (nu > 0) load_w(0, x0);
+    if (nu > 1) load_w(1, x1);
+  } else {
+    if (nub > 0) load_wb(0, y0);
+    if (DEPTH == 3 && nub > 1) load_wb(1, y1);
+  }
   if (!wait()) return;
-  if (nu > 0) load_m(0, x0);
-  if (nu > 1) load_m(1, x1);
+  if constexpr (mx) {
+    if (nu > 0) load_m(0, x0);
+    if (nu > 1) load_m(1, x1);
+  } else {
+    if (nub > 0) load_mb(0, y0);
+    if (DEPTH == 3 && nub > 1) load_mb(1, y1);
+  }
   down_shared<NW, NCG, DT>(p, t, KB2s, wave, lane, shraw, shsc, acc);
   if constexpr (mx) {
     auto step = [&](int u, Unit& cur, Unit& nxt2) {
@@ -1302,91 +1402,24 @@ MK2_DEV void down_rows(const MoeDev& p, int nt, float* red, int* act_ids, float*
       step(u + 1, x1, x0);
       step(u + 2, x2, x1);
     }
-  } else if constexpr (DT == 1) {
-    if constexpr (FMT == MK2_FMT_A16W4) {
-      // E2M1 weights widened exactly to bf16 against the bf16 mid, 8 k-blocks a batch
-      constexpr int KMAX = 8;
-      for (int j = wave; j < D; j += NW) {
-        const int e = act_ids[j];
-        const uint8_t* wb = p.w2 + ((size_t)e * HT + tl[0]) * KB2 * 1024;
-        const uint8_t* sb = p.s2 + e * e8m0_expert_bytes(p.wl, p.H, p.I);
-        f32x4 t[NCG];
-#pragma unroll
-        for (int cg = 0; cg < NCG; ++cg) t[cg] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int kb0 = 0; kb0 < KB2; kb0 += KMAX) {
-          uint4 raw[KMAX];
-          uint32_t sw[KMAX];
-#pragma unroll
-          for (int u = 0; u < KMAX; ++u) {
-            const int kb = min(kb0 + u, KB2 - 1);
-            raw[u] = ld_stream16(wb + ((size_t)kb * 64 + lane) * 16);
-            sw[u] = (e8m0_word(sb, p.wl, p.I, tl[0], kb, lane) >> e8m0_shift(p.wl, tl[0], kb)) & 0xFFu;
-          }
-#pragma unroll
-          for (int u = 0; u < KMAX; ++u) {
-            const int kb = kb0 + u;
-            if (kb >= KB2) break;
-            const float sc = e8m0_to_f32(sw[u]);
-            bf16x8 a[4];
-            a[0] = e2m1x8_to_bf16(raw[u].x, sc);
-            a[1] = e2m1x8_to_bf16(raw[u].y, sc);
-            a[2] = e2m1x8_to_bf16(raw[u].z, sc);
-            a[3] = e2m1x8_to_bf16(raw[u].w, sc);
-#pragma unroll
-            for (int cg = 0; cg < NCG; ++cg) {
-              bf16x8 b[4];
-              load_b_bf16(p.mid_b + (size_t)j * p.M * p.I, cg * 16 + c16, p.M, p.I, kb * 128 + 32 * g, b);
-              t[cg] = mfma4_bf16(a, b, t[cg]);
-            }
-          }
-        }
-#pragma unroll
-        for (int cg = 0; cg < NCG; ++cg) acc[0][cg] += t[cg] * ldp_f32(p.rw + j * 32 + cg * 16 + c16);
+  } else {
+    auto step = [&](int u, UnitB& cur, UnitB& nxt) {
+      if (u + DEPTH - 1 < nub) {
+        load_wb(u + DEPTH - 1, nxt);
+        load_mb(u + DEPTH - 1, nxt);
+      }
+      if (u < nub) compute_b(u, cur);
+    };
+    if constexpr (DEPTH == 3) {
+      for (int u = 0; u < nub; u += 3) {
+        step(u, y0, y2);
+        step(u + 1, y1, y0);
+        step(u + 2, y2, y1);
       }
     } else {
-      // E4M3 weights (f32 scale per 128 x 128 block): widened to bf16 against the bf16
-      // mid (W8A16), or on the scaled MFMA against the E4M3 mid (W8A8, f32 scale per 128
-      // a row); each k-block's product times its scales and the route weight
-      constexpr int KMAX = 8;  // inter <= 1024
-      constexpr bool w8a8 = FMT == MK2_FMT_W8A8;
-      for (int j = wave; j < D; j += NW) {
-        const int e = act_ids[j];
-        const uint8_t* wb = p.w2 + ((size_t)e * HT + tl[0]) * KB2 * 2048;
-        const float* sbase = (const float*)p.s2 + (size_t)e * (p.H / 128) * KB2 + (tl[0] * 16 / 128) * KB2;
-        uint4 raw[KMAX][2];
-#pragma unroll
-        for (int kb = 0; kb < KMAX; ++kb) {
-          load_fp8_block(wb + (size_t)min(kb, KB2 - 1) * 2048, p.wl, lane, raw[kb][0], raw[kb][1]);
-        }
-#pragma unroll
-        for (int kb = 0; kb < KMAX; ++kb) {
-          if (kb >= KB2) break;
-          const float sc = sbase[kb];
-          if constexpr (w8a8) {
-            const i32x8 A = {(int)raw[kb][0].x, (int)raw[kb][0].y, (int)raw[kb][0].z, (int)raw[kb][0].w,
-                             (int)raw[kb][1].x, (int)raw[kb][1].y, (int)raw[kb][1].z, (int)raw[kb][1].w};
-#pragma unroll
-            for (int cg = 0; cg < NCG; ++cg) {
-              const int row = cg * 16 + c16;
-              const i32x8 bq = load_b_fp8_same(p.mid_q + (size_t)j * p.M * p.I, row, p.M, p.I, kb * 128, g);
-              const float ms = row < p.M ? ldp_f32(p.mid_sf + ((size_t)j * p.M + row) * (p.I / 128) + kb) : 0.f;
-              acc[0][cg] += mfma_same<0>(A, bq, f32x4{0.f, 0.f, 0.f, 0.f}, E8M0_ONE, E8M0_ONE) *
-                            (sc * ms * ldp_f32(p.rw + j * 32 + row));
-            }
-          } else {
-            bf16x8 a[4];
-            a[0] = e4m3x8_to_bf16(raw[kb][0].x, raw[kb][0].y);
-            a[1] = e4m3x8_to_bf16(raw[kb][0].z, raw[kb][0].w);
-            a[2] = e4m3x8_to_bf16(raw[kb][1].x, raw[kb][1].y);
-            a[3] = e4m3x8_to_bf16(raw[kb][1].z, raw[kb][1].w);
-#pragma unroll
-            for (int cg = 0; cg < NCG; ++cg) {
-              bf16x8 b[4];
-              load_b_bf16(p.mid_b + (size_t)j * p.M * p.I, cg * 16 + c16, p.M, p.I, kb * 128 + 32 * g, b);
-              acc[0][cg] += mfma4_bf16(a, b, f32x4{0.f, 0.f, 0.f, 0.f}) * (sc * ldp_f32(p.rw + j * 32 + cg * 16 + c16));
-            }
-          }
-        }
+      for (int u = 0; u < nub; u += 2) {
+        step(u, y0, y1);
+        step(u + 1, y1, y0);
       }
     }
   }
@@ -1631,8 +1664,22 @@ MK2_DEV void down_rows_cmp(const MoeDev& p, int nt, float* red, int* act_ids, fl
   __syncthreads();
 }
 
-// down tasks of a launch: 16 * DT hidden rows each, or 24 with DT == 3
-__host__ __device__ inline int down_tasks(const MoeDev& p) { return p.DT == 3 ? p.H / 24 : p.H / (16 * p.DT); }
+// The hidden rows of a down task, 16, 24 or 32 (a divisor of H), for the 256 workgroups of
+// MI355X: the busiest workgroup's rounds times a task's cost, its rows plus about 8 rows'
+// worth of mid loads and hand-offs.  2048, 3072 and 4096 -> 16 (128, 192, 256 tasks), 6144 ->
+// 24 (256), 7168 -> 32 (224).  A8W4 at 2048, 8 rows (128 experts of 768): 62.0 -> 56.4 us in
+// 16-row tasks instead of 32; 8-row tasks took 59.3 (half-empty tiles, twice the mid loads).
+inline int down_task_rows(int H) {
+  int best = 16, cost = 1 << 30;
+  for (const int rows : {32, 24, 16}) {
+    if (H % rows) continue;
+    const int c = (H / rows + 255) / 256 * (rows + 8);
+    if (c < cost) cost = c, best = rows;
+  }
+  return best;
+}
+// down tasks of a launch
+__host__ __device__ inline int down_tasks(const MoeDev& p) { return p.H / p.DR; }
 
 // task nt of down_tasks(p).  Needs the routing (act, rw) on entry; `wait` is the
 // mid activations' dependency, run once the task's static and routed weight loads
@@ -1640,18 +1687,11 @@ __host__ __device__ inline int down_tasks(const MoeDev& p) { return p.DT == 3 ? 
 template <int NT, int NCG, int FMT, typename Wait = NoWait>
 MK2_DEV void moe_down(const MoeDev& p, int nt, float* red, int* act_ids, float* xres, Wait wait = Wait()) {
   if constexpr (kCompact<NCG, FMT>) {
-    // 24 hidden rows a task where hidden is a multiple of 48 (one task a CU at 6144),
-    // else 16
-    if (p.DT == 3) down_rows_cmp<NT, NCG, 2, FMT>(p, nt, red, act_ids, xres, wait);
+    if (p.DR > 16) down_rows_cmp<NT, NCG, 2, FMT>(p, nt, red, act_ids, xres, wait);
     else down_rows_cmp<NT, NCG, 1, FMT>(p, nt, red, act_ids, xres, wait);
   } else {
-    if constexpr (FMT == MK2_FMT_MXFP4 || FMT == MK2_FMT_A4W4) {
-      if (NCG == 1 && p.DT >= 2) {
-        down_rows<NT, NCG, (NCG == 1 ? 2 : 1), FMT>(p, nt, red, act_ids, xres, wait);
-        return;
-      }
-    }
-    down_rows<NT, NCG, 1, FMT>(p, nt, red, act_ids, xres, wait);
+    if (p.DR > 16) down_rows<NT, NCG, 2, FMT>(p, nt, red, act_ids, xres, wait);
+    else down_rows<NT, NCG, 1, FMT>(p, nt, red, act_ids, xres, wait);
   }
 }
 

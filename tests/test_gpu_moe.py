@@ -111,14 +111,28 @@ def test_moe_mxfp4_config2(rows):
 
 @pytest.mark.parametrize("hidden", [2048, 7168])
 def test_moe_mxfp4_down_tiles(hidden):
-    """Down tasks of 32 hidden rows (hidden not a multiple of 48; 6144 takes 24-row
-    tasks), with the norm and the residual."""
+    """Down tasks of 16 and 32 hidden rows (6144 takes 24-row tasks), with the norm and the
+    residual."""
     from dataclasses import replace
 
     from sgl_amd_mono.k2 import config as C
 
     cfg = replace(C.C2_MOE, hidden=hidden, n_experts=64)
     w, out, logits, ids, wts = _run(cfg, 8, seed=hidden, norm=True, residual=True)
+    _check(cfg, w, out, logits, ids, wts, norm=True, residual=True)
+
+
+@pytest.mark.parametrize("fmt", ["FP8", "W8A8", "A16W4"])
+@pytest.mark.parametrize("hidden, inter, rows", [(6144, 128, 3), (2048, 384, 17), (7168, 384, 20), (6144, 256, 16)])
+def test_moe_down_pipeline(fmt, hidden, inter, rows):
+    """The slot pipeline of the bf16-mid and W8A8 downs: one k-block a slot, odd numbers of
+    them, 16-, 24- and 32-row tasks, one and two column groups."""
+    from dataclasses import replace
+
+    from sgl_amd_mono.k2 import config as C
+
+    cfg = replace(C.C2_MOE, hidden=hidden, inter=inter, n_experts=64, expert_fmt=getattr(C, "FMT_" + fmt))
+    w, out, logits, ids, wts = _run(cfg, rows, seed=hidden + inter + rows, norm=True, residual=True)
     _check(cfg, w, out, logits, ids, wts, norm=True, residual=True)
 
 
