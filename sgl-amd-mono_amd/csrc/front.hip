@@ -39,15 +39,21 @@
 
 namespace mk2 {
 
-template <int KU, int WF>
+template <int KU, int WF, int NCG>
 __global__ __launch_bounds__(GV_NT) void k_gemv(GemvDev p) {
   __shared__ GemvLds S;
-  gemv_run<KU, WF>(p, blockIdx.x, gridDim.x, S);
+  gemv_run<KU, WF, NCG>(p, blockIdx.x, gridDim.x, S);
 }
 
 template <int KU, int WF>
 static void gemv_launch1(const GemvDev& d, int grid, hipStream_t st) {
-  k_gemv<KU, WF><<<grid, GV_NT, 0, st>>>(d);
+  if constexpr (KU <= GV_KU2) {
+    if (d.M > 16) {
+      k_gemv<KU, WF, 2><<<grid, GV_NT, 0, st>>>(d);
+      return;
+    }
+  }
+  k_gemv<KU, WF, 1><<<grid, GV_NT, 0, st>>>(d);
 }
 
 // the engine's k-step counts: KU = K / (512 ks)
@@ -106,7 +112,7 @@ __global__ __launch_bounds__(FR_NT) void k_front_heads(FrontDev p) {
 }
 
 
-template <int KUA, int KUC, int WF, int NS>
+template <int KUA, int KUC, int WF, int NS, int NCG>
 __global__ __launch_bounds__(FR_NT, 1) void k_front_persistent(FrontPDev p) {
   __shared__ FrontLds S;
   __shared__ int seen[FP_SEEN];
@@ -114,7 +120,7 @@ __global__ __launch_bounds__(FR_NT, 1) void k_front_persistent(FrontPDev p) {
   const int G = gridDim.x;
   if (threadIdx.x < FP_SEEN) seen[threadIdx.x] = 0;
   __syncthreads();
-  front_walk<KUA, KUC, WF, NS>(p, S, seen);
+  front_walk<KUA, KUC, WF, NS, NCG>(p, S, seen);
   // the last workgroup out resets the counters for the next launch
   drain_memory();
   __syncthreads();
@@ -233,23 +239,24 @@ static bool front_persistent_ok(const mk2_front_shape* s) {
 #undef MK2_FP_MATCH
 }
 
-template <int KUA, int KUC, int WF, int NS>
+template <int KUA, int KUC, int WF, int NS, int NCG>
 static int front_persistent_launch(const FrontPDev& d, int cus, hipStream_t st) {
   static int fits = -1;  // one workgroup a CU
   if (fits < 0) {
     int per_cu = 0;
-    fits = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_front_persistent<KUA, KUC, WF, NS>, FR_NT, 0) ==
+    fits = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_front_persistent<KUA, KUC, WF, NS, NCG>, FR_NT, 0) ==
                    hipSuccess &&
            per_cu >= 1;
   }
   if (!fits) return set_error(MK2_ELAUNCH, "front: the persistent kernel does not fit one workgroup per CU");
-  k_front_persistent<KUA, KUC, WF, NS><<<cus, FR_NT, 0, st>>>(d);
+  k_front_persistent<KUA, KUC, WF, NS, NCG><<<cus, FR_NT, 0, st>>>(d);
   return check_launch("front (persistent)");
 }
 
 static int front_persistent_dispatch(const FrontPDev& d, int wf, const FrontSteps& k, int cus, hipStream_t st) {
 #define MK2_FP_CASE(WF, A, C, N) \
-  if (wf == WF && k.kua == A && k.kuc == C && k.ns == N) return front_persistent_launch<A, C, WF, N>(d, cus, st);
+  if (wf == WF && k.kua == A && k.kuc == C && k.ns == N)        \
+    return d.f.M > 16 ? front_persistent_launch<A, C, WF, N, 2>(d, cus, st) : front_persistent_launch<A, C, WF, N, 1>(d, cus, st);
   MK2_FRONT_PERSISTENT_SHAPES(MK2_FP_CASE, MK2_WFMT_BF16)
   MK2_FRONT_PERSISTENT_SHAPES(MK2_FP_CASE, MK2_WFMT_FP8_BLOCK)
   MK2_FRONT_PERSISTENT_SHAPES(MK2_FP_CASE, MK2_WFMT_FP8_AITER16)
@@ -305,15 +312,19 @@ static int front_prepare(const mk2_front_args* a, FrontPrep* P) {
   auto seg = [](const void* w, const float* sc, float* out, int rows, int ld, long long pstride) {
     return GemvSeg{w, sc, out, rows, ld, pstride};
   };
-  // the GEMV passes of 16 rows: hidden-input [W_qkv_a | W_ik] and W_iw, q_an-input
-  // [W_q_b | W_iq]
-  const int passes = P->passes = (M + 15) / 16;
+  // the GEMV passes: hidden-input [W_qkv_a | W_ik] and W_iw, q_an-input [W_q_b | W_iq].  Up to
+  // 32 rows are one pass where the engine's two column groups fit the slices (every shape
+  // of the persistent launch); else passes of 16.  Two passes read the weights twice: C7 at
+  // 32 rows took 49.3 us, one takes 40.6 (17 rows 41.2 -> 34.0, bf16 weights at 32 61.7 -> 46.8)
+  const FrontSteps fs = front_steps(&s);
+  const int wide = fs.kua <= GV_KU2 && fs.kuc <= GV_KU2 && (!idx || fs.kuw <= GV_KU2) ? 32 : 16;
+  const int passes = P->passes = (M + wide - 1) / wide;
   for (int pi = 0; pi < 2; ++pi) P->gA[pi] = P->gW[pi] = P->gC[pi] = GemvDev{};
   for (int pi = 0; pi < passes; ++pi) {
-    const int r0 = 16 * pi;
+    const int r0 = wide * pi;
     GemvDev& d = P->gA[pi];
-    d.M = M - r0 < 16 ? M - r0 : 16; d.K = s.hidden; d.ks = pl.ksA; d.eps = s.eps;
-    d.x = ws.x_n + (size_t)r0 * s.hidden; d.g = nullptr;
+    d.M = M - r0 < wide ? M - r0 : wide; d.K = s.hidden; d.ks = pl.ksA;
+    d.x = ws.x_n + (size_t)r0 * s.hidden;
     d.seg[0] = seg(w.w_qkv_a, w.s_qkv_a, ws.qkv_a + (size_t)r0 * NA, NA, NA, (long long)M * NA);
     d.tiles0 = NA / 16; d.ntiles = d.tiles0;
     if (idx) {
@@ -326,8 +337,8 @@ static int front_prepare(const mk2_front_args* a, FrontPrep* P) {
       e.tiles0 = IH / 16; e.ntiles = e.tiles0;
     }
     GemvDev& c = P->gC[pi];
-    c.M = d.M; c.K = s.q_lora; c.ks = pl.ksC; c.eps = s.eps;
-    c.x = ws.q_an + (size_t)r0 * s.q_lora; c.g = nullptr;
+    c.M = d.M; c.K = s.q_lora; c.ks = pl.ksC;
+    c.x = ws.q_an + (size_t)r0 * s.q_lora;
     c.seg[0] = seg(w.w_q_b, w.s_q_b, ws.q_b + (size_t)r0 * QB, QB, QB, (long long)M * QB);
     c.tiles0 = QB / 16; c.ntiles = c.tiles0;
     if (idx) {

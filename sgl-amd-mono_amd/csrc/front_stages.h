@@ -10,8 +10,9 @@ namespace mk2 {
 
 constexpr int GV_NT = 512;
 constexpr int GV_WAVES = GV_NT / 64;
-constexpr int GV_CHUNK = 8;  // tiles whose partials wait in LDS for one barrier
+constexpr int GV_CHUNK = 8;  // tiles and column groups whose partials wait in LDS for one barrier
 constexpr int FR_NT = 512;
+constexpr int GV_KU2 = 8;    // the longest slice (64-k units a wave) two column groups take
 
 struct GemvSeg {
   const void* w;   // [rows][K] bf16 or E4M3, row-major
@@ -23,38 +24,35 @@ struct GemvSeg {
 };
 
 struct GemvDev {
-  int M;   // rows this pass, 1..16
+  int M;   // rows this pass, 1..16 NCG
   int K;
   int ks;  // K parts: workgroup b takes part b % ks (the grid is a multiple of ks)
-  float eps;
-  const bf16_t* x;  // [M][K]: raw rows (with g) or the GEMV input as it is (g null)
-  const bf16_t* g;  // RMSNorm weight [K], or null
+  const bf16_t* x;  // [M][K]
   GemvSeg seg[2];
   int tiles0;  // 16-row tiles of segment 0
   int ntiles;
 };
 
 struct GemvLds {
-  float ssum[16];
-  uint4 gam[8192 / 8];
   float red[GV_CHUNK][GV_WAVES][256];
 };
 
 // One engine workgroup's work: workgroup b of nblocks (a multiple of p.ks).  KU: 64-k
 // units a wave (K / ks = 8 * 64 * KU); WF: the weights' MK2_WFMT_* (bf16, E4M3
-// row-major, or E4M3 in AITER's (16, 16) layout).  `wait` (the input rows'
+// row-major, or E4M3 in AITER's (16, 16) layout); NCG: column groups of 16 rows, so that
+// 32 rows take one pass over the weights.  `wait` (the input rows'
 // dependency, in the persistent front) runs once the first tile's weights are in
 // flight; false from it returns false at once.  The f32 partial planes are stored
 // device-coherently (the next stage may run on another XCD within the same launch).
-template <int KU, int WF, typename Wait = NoWait>
+template <int KU, int WF, int NCG, typename Wait = NoWait>
 MK2_DEV bool gemv_run(const GemvDev& p, int b, int nblocks, GemvLds& S, Wait wait = Wait()) {
   constexpr bool F8 = WF != MK2_WFMT_BF16, SHUF = WF == MK2_WFMT_FP8_AITER16;
   constexpr int L = F8 ? KU : 2 * KU;      // 16-byte weight loads a lane a tile
   constexpr int WIN = L <= 24 ? L : L / 2;  // loads in flight a lane
   static_assert(L % WIN == 0, "a window divides the loads of a tile");
   static_assert(!F8 || KU % 2 == 0, "FP8 slices are whole 128-k blocks");
-  float* ssum = S.ssum;
-  uint4* gam = S.gam;
+  static_assert(NCG == 1 || KU <= GV_KU2, "two groups' operands fit the registers");
+  constexpr int CH = GV_CHUNK / NCG;  // tiles a barrier phase
   auto& red = S.red;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, g = lane >> 4;
   const int K = p.K, M = p.M;
@@ -63,7 +61,6 @@ MK2_DEV bool gemv_run(const GemvDev& p, int b, int nblocks, GemvLds& S, Wait wai
   // k map: unit u of the wave's slice holds k = kw + 64 u + 0 .. 15 for lane group g;
   // MFMA step 2u takes its first 8, step 2u + 1 the next 8 (A and B alike)
   const int kw = part * (K / p.ks) + wave * KU * 64 + 16 * g;
-  const bool live = c16 < M;
   // the tile sequence: tile t of segment sid at row (t - base) * 16; this lane's row
   auto seg_of = [&](int t) { return t < p.tiles0 ? 0 : 1; };
   // In AITER's (16, 16) layout ([rows/16][K/32][2][16 rows][16 B]) the 16 bytes of
@@ -85,85 +82,51 @@ MK2_DEV bool gemv_run(const GemvDev& p, int b, int nblocks, GemvLds& S, Wait wai
     for (int j = 0; j < WIN; ++j) wv[j] = ld_stream16(wrow + w_off(j));
   }
   if (!wait()) return false;
-  // the rows: this lane's fragments of row c16 (16 k a unit)
-  const bf16_t* xr = p.x + (size_t)(live ? c16 : 0) * K + kw;
-  uint4 xq[2 * KU];
+  // B operands: this lane's fragments of rows 16 cg + c16 (16 k a unit), zero past the rows
+  bf16x8 bq[NCG][2 * KU];
 #pragma unroll
-  for (int u = 0; u < KU; ++u) {
-    xq[2 * u] = *(const uint4*)(xr + 64 * u);
-    xq[2 * u + 1] = *(const uint4*)(xr + 64 * u + 8);
-  }
-  // the norm: each row's sum of squares over all K (the rows are L2-resident): 32
-  // threads a row, 16-byte pieces, every load issued before the sums
-  float rs = 1.f;
-  if (p.g) {
-    constexpr int PB = 12;  // pieces a thread a batch
-    const int mr = threadIdx.x >> 5, tr = threadIdx.x & 31;
-    const uint4* xrow = (const uint4*)(p.x + (size_t)(mr < M ? mr : 0) * K);
-    float ss = 0.f;
-    for (int i0 = tr; i0 < K / 8; i0 += 32 * PB) {
-      uint4 v[PB];
+  for (int cg = 0; cg < NCG; ++cg) {
+    const bool live = 16 * cg + c16 < M;
+    const bf16_t* xr = p.x + (size_t)(live ? 16 * cg + c16 : 0) * K + kw;
+    uint4 xq[2 * KU];
 #pragma unroll
-      for (int j = 0; j < PB; ++j) v[j] = i0 + 32 * j < K / 8 ? xrow[i0 + 32 * j] : make_uint4(0, 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < PB; ++j) {
-        const uint32_t u4[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const bf16x2 h = __builtin_bit_cast(bf16x2, u4[e]);
-          ss = __builtin_amdgcn_fdot2_f32_bf16(h, h, ss, false);
-        }
-      }
+    for (int u = 0; u < KU; ++u) {
+      xq[2 * u] = *(const uint4*)(xr + 64 * u);
+      xq[2 * u + 1] = *(const uint4*)(xr + 64 * u + 8);
     }
 #pragma unroll
-    for (int m = 1; m < 32; m <<= 1) ss += __shfl_xor(ss, m);
-    if (tr == 0 && mr < M) ssum[mr] = ss;
-    for (int j = threadIdx.x; j < K / 8; j += GV_NT) gam[j] = ((const uint4*)p.g)[j];
-    __syncthreads();
-    rs = live ? 1.0f / sqrtf(ssum[c16] / (float)K + p.eps) : 0.f;
+    for (int i = 0; i < 2 * KU; ++i) bq[cg][i] = __builtin_bit_cast(bf16x8, live ? xq[i] : make_uint4(0, 0, 0, 0));
   }
-  // B operands: bf16(x * rstd * g), or x as it is; zero columns past the rows
-  bf16x8 bq[2 * KU];
+  // the tiles, in chunks of CH whose partials wait in LDS (no barrier a tile)
+  for (int c0 = t0; c0 < t1; c0 += CH) {
 #pragma unroll
-  for (int i = 0; i < 2 * KU; ++i) {
-    uint4 ov = xq[i];
-    if (p.g) {
-      const uint4 gv = gam[(kw + 64 * (i >> 1) + 8 * (i & 1)) >> 3];
-      const uint32_t xu[4] = {xq[i].x, xq[i].y, xq[i].z, xq[i].w}, gu[4] = {gv.x, gv.y, gv.z, gv.w};
-      uint32_t o[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        o[j] = pack_bf16x2(__uint_as_float(xu[j] << 16) * rs * __uint_as_float(gu[j] << 16),
-                           __uint_as_float(xu[j] & 0xFFFF0000u) * rs * __uint_as_float(gu[j] & 0xFFFF0000u));
-      ov = make_uint4(o[0], o[1], o[2], o[3]);
-    }
-    if (!live) ov = make_uint4(0, 0, 0, 0);
-    bq[i] = __builtin_bit_cast(bf16x8, ov);
-  }
-  // the tiles, in chunks of GV_CHUNK whose partials wait in LDS (no barrier a tile)
-  for (int c0 = t0; c0 < t1; c0 += GV_CHUNK) {
-#pragma unroll
-    for (int i = 0; i < GV_CHUNK; ++i) {
+    for (int i = 0; i < CH; ++i) {
       const int t = c0 + i;
       if (t >= t1) break;
       const bool more = t + 1 < t1;
       const uint8_t* nrow = w_row(more ? t + 1 : t);
       const int sid = seg_of(t);
       const int row0 = (t - (sid ? p.tiles0 : 0)) * 16;
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      f32x4 acc[NCG];
+#pragma unroll
+      for (int cg = 0; cg < NCG; ++cg) acc[cg] = f32x4{0.f, 0.f, 0.f, 0.f};
       if constexpr (F8) {
         // the tile's block scales (one a 128-k block of the wave's slice; the tile's 16
         // rows are in one 128-row block)
         const float* sr = p.seg[sid].s + (size_t)(row0 >> 7) * (K >> 7) + ((kw - 16 * g) >> 7);
 #pragma unroll
         for (int kb = 0; kb < KU / 2; ++kb) {
-          f32x4 pa = {0.f, 0.f, 0.f, 0.f};
+          f32x4 pa[NCG];
+#pragma unroll
+          for (int cg = 0; cg < NCG; ++cg) pa[cg] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
             const int j = 2 * kb + h;
-            const uint4 w = wv[j % WIN];
-            pa = mfma_bf16(e4m3x8_to_bf16(w.x, w.y), bq[2 * j], pa);
-            pa = mfma_bf16(e4m3x8_to_bf16(w.z, w.w), bq[2 * j + 1], pa);
+            const bf16x8 w0 = e4m3x8_to_bf16(wv[j % WIN].x, wv[j % WIN].y), w1 = e4m3x8_to_bf16(wv[j % WIN].z, wv[j % WIN].w);
+#pragma unroll
+            for (int cg = 0; cg < NCG; ++cg) pa[cg] = mfma_bf16(w0, bq[cg][2 * j], pa[cg]);
+#pragma unroll
+            for (int cg = 0; cg < NCG; ++cg) pa[cg] = mfma_bf16(w1, bq[cg][2 * j + 1], pa[cg]);
             const int nj = j + WIN;
             if (nj < L)
               wv[j % WIN] = ld_stream16(wrow + w_off(nj));
@@ -172,12 +135,15 @@ MK2_DEV bool gemv_run(const GemvDev& p, int b, int nblocks, GemvLds& S, Wait wai
           }
           const float sc = sr[kb];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[e] += pa[e] * sc;
+          for (int cg = 0; cg < NCG; ++cg)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[cg][e] += pa[cg][e] * sc;
         }
       } else {
 #pragma unroll
         for (int j = 0; j < L; ++j) {
-          acc = mfma_bf16(__builtin_bit_cast(bf16x8, wv[j % WIN]), bq[j], acc);
+#pragma unroll
+          for (int cg = 0; cg < NCG; ++cg) acc[cg] = mfma_bf16(__builtin_bit_cast(bf16x8, wv[j % WIN]), bq[cg][j], acc[cg]);
           const int nj = j + WIN;
           if (nj < L)
             wv[j % WIN] = ld_stream16(wrow + w_off(nj));
@@ -186,20 +152,21 @@ MK2_DEV bool gemv_run(const GemvDev& p, int b, int nblocks, GemvLds& S, Wait wai
         }
       }
       // lane (c16, g) holds D[v = 4 g + e][m = c16]
-      float* rw = red[i][wave];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) rw[(4 * g + e) * 16 + c16] = acc[e];
+      for (int cg = 0; cg < NCG; ++cg)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red[i * NCG + cg][wave][(4 * g + e) * 16 + c16] = acc[cg][e];
       wrow = nrow;
     }
     __syncthreads();
-    const int nt = min(GV_CHUNK, t1 - c0);
-    for (int e = threadIdx.x; e < nt * 256; e += GV_NT) {
-      const int i = e >> 8, m = (e >> 4) & 15, v = e & 15;
-      const int t = c0 + i, sid = seg_of(t);
+    const int nt = min(CH, t1 - c0);
+    for (int e = threadIdx.x; e < nt * NCG * 256; e += GV_NT) {
+      const int i = e >> 8, m16 = (e >> 4) & 15, v = e & 15, m = i % NCG * 16 + m16;
+      const int t = c0 + i / NCG, sid = seg_of(t);
       const int row = (t - (sid ? p.tiles0 : 0)) * 16 + v;
-      float s = red[i][0][v * 16 + m];
+      float s = red[i][0][v * 16 + m16];
 #pragma unroll
-      for (int w = 1; w < GV_WAVES; ++w) s += red[i][w][v * 16 + m];
+      for (int w = 1; w < GV_WAVES; ++w) s += red[i][w][v * 16 + m16];
       if (m < M) st_dev_f32(p.seg[sid].out + part * p.seg[sid].pstride + (size_t)m * p.seg[sid].ld + row, s);
     }
     __syncthreads();
@@ -578,7 +545,7 @@ static_assert(FP_STATUS * FP_LINE * 4 == MK2_FRONT_STATUS_OFFSET, "the status wo
 
 struct FrontPDev {
   FrontDev f;
-  GemvDev A[2], W[2], C[2];  // passes of 16 rows
+  GemvDev A[2], W[2], C[2];  // by pass: the rows the engine takes at once (16 or 32)
   int passes, gridA, gridW, gridC, nheads;
   const bf16_t* x;
   const bf16_t* g_in;
@@ -656,7 +623,7 @@ MK2_DEV bool fp_wait(const FrontPDev& p, int* seen, int k, int line, int lanes, 
 // start.  With HEADS the per-head tasks also count out on FP_HEADS (the persistent
 // layer that runs the front ahead of its own stages waits on it); their outputs and
 // the cache rows are stored device-coherently either way.
-template <int KUA, int KUC, int WF, int NS, bool HEADS = false>
+template <int KUA, int KUC, int WF, int NS, int NCG, bool HEADS = false>
 MK2_DEV bool front_walk(const FrontPDev& p, FrontLds& S, int* seen) {
   const int G = gridDim.x, b = blockIdx.x, M = p.f.M;
   int base = 0;
@@ -668,13 +635,13 @@ MK2_DEV bool front_walk(const FrontPDev& p, FrontLds& S, int* seen) {
     fp_signal(p, FP_NORM, 0, 1);
   }
   FP_NEXT(M);
-  // 1. the hidden-input GEMVs, per pass of 16 rows: [W_qkv_a | W_ik], then W_iw
+  // 1. the hidden-input GEMVs, per pass: [W_qkv_a | W_ik], then W_iw
   const int nA = p.gridA + p.gridW;
   FP_TASKS(t, p.passes * nA) {
     const int pass = t / nA, u = t % nA;
     auto w = [&] { return fp_wait(p, seen, 0, FP_NORM, 1, M); };
-    const bool ok = u < p.gridA ? gemv_run<KUA, WF>(p.A[pass], u, p.gridA, S.gemv, w)
-                                : gemv_run<1, MK2_WFMT_BF16>(p.W[pass], u - p.gridA, p.gridW, S.gemv, w);
+    const bool ok = u < p.gridA ? gemv_run<KUA, WF, NCG>(p.A[pass], u, p.gridA, S.gemv, w)
+                                : gemv_run<1, MK2_WFMT_BF16, NCG>(p.W[pass], u - p.gridA, p.gridW, S.gemv, w);
     if (!ok) return false;
     fp_signal(p, FP_A, t, FP_LANES);
   }
@@ -690,7 +657,7 @@ MK2_DEV bool front_walk(const FrontPDev& p, FrontLds& S, int* seen) {
   // 3. the q_an-input GEMVs
   FP_TASKS(t, p.passes * p.gridC) {
     const int pass = t / p.gridC, u = t % p.gridC;
-    if (!gemv_run<KUC, WF>(p.C[pass], u, p.gridC, S.gemv, [&] { return fp_wait(p, seen, 2, FP_ROWS, FP_LANES, nR); }))
+    if (!gemv_run<KUC, WF, NCG>(p.C[pass], u, p.gridC, S.gemv, [&] { return fp_wait(p, seen, 2, FP_ROWS, FP_LANES, nR); }))
       return false;
     fp_signal(p, FP_C, t, FP_LANES);
   }

@@ -266,11 +266,11 @@ struct K2NoFront {
   MK2_DEV bool run(FrontLds&, int*) const { return true; }
   MK2_DEV void reset() const {}
 };
-template <int KUA, int KUC, int WF, int NS>
+template <int KUA, int KUC, int WF, int NS, int NCG>
 struct K2Front {
   FrontPDev f;
   MK2_DEV bool run(FrontLds& S, int* seen) const {
-    if (!front_walk<KUA, KUC, WF, NS, true>(f, S, seen)) return false;
+    if (!front_walk<KUA, KUC, WF, NS, NCG, true>(f, S, seen)) return false;
     return fp_wait(f, seen, 4, FP_HEADS, FP_LANES, f.nheads);
   }
   MK2_DEV void reset() const { front_reset(f); }
@@ -565,21 +565,23 @@ int k2_persistent_enqueue(const IdxDev& idx, const MlaDev& mla, const MoeDev& mo
   // front shape)
   return with_moe_fmt(moe.fmt, [&](auto F) {
     constexpr int FMT = decltype(F)::value;
-    auto launch = [&](auto fr) -> int {
-      using Fr = decltype(fr);
+    auto launch = [&](auto kern, auto fr) -> int {
       int per_cu = 0;
-      hipError_t e = two ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_k2_layer<2, FMT, Fr>, K2_NT, 0)
-                         : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_k2_layer<1, FMT, Fr>, K2_NT, 0);
-      if (e != hipSuccess || per_cu < 1)
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, K2_NT, 0) != hipSuccess || per_cu < 1)
         return set_error(MK2_ELAUNCH, "layer: the persistent kernel does not fit one workgroup per CU");
-      if (two) k_k2_layer<2, FMT, Fr><<<ncu, K2_NT, 0, st>>>(p, fr);
-      else k_k2_layer<1, FMT, Fr><<<ncu, K2_NT, 0, st>>>(p, fr);
+      kern<<<ncu, K2_NT, 0, st>>>(p, fr);
       return check_launch("layer (persistent)");
     };
-    if (!front) return launch(K2NoFront{});
+    if (!front)
+      return two ? launch(k_k2_layer<2, FMT, K2NoFront>, K2NoFront{}) : launch(k_k2_layer<1, FMT, K2NoFront>, K2NoFront{});
     if constexpr (FMT == MK2_FMT_MXFP4) {
-      if (front_key == FRONT_FUSED_C7_FP8) return launch(K2Front<6, 4, MK2_WFMT_FP8_BLOCK, 6>{*front});
-      if (front_key == FRONT_FUSED_C7_AITER16) return launch(K2Front<6, 4, MK2_WFMT_FP8_AITER16, 6>{*front});
+      auto with = [&](auto WF) -> int {
+        using F1 = K2Front<6, 4, decltype(WF)::value, 6, 1>;
+        using F2 = K2Front<6, 4, decltype(WF)::value, 6, 2>;
+        return two ? launch(k_k2_layer<2, FMT, F2>, F2{*front}) : launch(k_k2_layer<1, FMT, F1>, F1{*front});
+      };
+      if (front_key == FRONT_FUSED_C7_FP8) return with(std::integral_constant<int, MK2_WFMT_FP8_BLOCK>{});
+      if (front_key == FRONT_FUSED_C7_AITER16) return with(std::integral_constant<int, MK2_WFMT_FP8_AITER16>{});
     }
     return set_error(MK2_EINVAL, "layer step: no front-and-layer launch for this expert mode and front shape");
   });

@@ -272,3 +272,38 @@ def test_front_persistent_new_inputs_each_launch():
     assert p_op.status() == 0
     assert not torch.equal(outs[0], outs[1])
     assert torch.equal(outs[0], outs[2]) and torch.equal(outs[1], outs[3])
+
+
+@pytest.mark.parametrize("wfmt, hidden, q_lora, heads, index_heads, rows",
+                         [("FP8_BLOCK", 6144, 2048, 16, 64, 17), ("FP8_AITER16", 6144, 2048, 16, 64, 32),
+                          ("BF16", 7168, 2048, 16, 32, 27), ("FP8_BLOCK", 4096, 1024, 32, 0, 31),
+                          ("BF16", 8192, 8192, 16, 16, 19)])
+def test_front_above_16_rows_matches_narrow_calls(wfmt, hidden, q_lora, heads, index_heads, rows):
+    """Above 16 rows the GEMVs take two column groups in one pass over the weights (two
+    passes where a slice is too long: the last shape): the bits of the same rows in two
+    calls, outputs and cache rows alike."""
+    from dataclasses import replace
+
+    from sgl_amd_mono.k2 import config as C, synth
+    from sgl_amd_mono.k2.ops import FrontOp
+
+    dev = torch.device("cuda:0") if torch.cuda.is_available() else pytest.skip("no GPU")
+    fmt = getattr(C, "WFMT_" + wfmt)
+    base = C.WFMT_FP8_BLOCK if fmt == C.WFMT_FP8_AITER16 else fmt
+    cfg = C.FrontConfig(hidden=hidden, q_lora=q_lora, heads=heads, index_heads=index_heads, weight_fmt=base,
+                        max_position=4095)
+    ns = synth.make_front(cfg, rows, hidden + rows, dev)
+    if fmt != base:
+        ns, cfg = synth.front_in_layout(ns, fmt), replace(cfg, weight_fmt=fmt)
+
+    def run(spans):
+        caches = [t.clone() if t is not None else None for t in (ns.kv_cache, ns.kv_scale, ns.index_cache, ns.index_scale)]
+        outs = []
+        for a, b in spans:
+            op = FrontOp(cfg, ns, b - a, dev)
+            outs.append(op(ns.x[a:b].contiguous(), ns.positions[a:b].contiguous(), ns.slots[a:b].contiguous(),
+                           ns.rope_cos_sin, *caches))
+        return [torch.cat(t) for t in zip(*outs) if t[0] is not None] + [t for t in caches if t is not None]
+
+    for x, y in zip(run([(0, rows)]), run([(0, 16), (16, rows)])):
+        assert torch.equal(x, y)
