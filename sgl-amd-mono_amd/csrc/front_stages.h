@@ -520,26 +520,35 @@ MK2_DEV bool front_heads_task(const FrontDev& p, int b, uint4* qn, Wait wait = W
 // stage's base continuing from the previous stage's last task, and a task that needs
 // an earlier stage's results waits on that stage's completion counter, as the
 // persistent layer does: producers store their hand-off data device-coherently,
-// drain, pass a barrier and add to the counter (16 sub-counters on their own lines
-// for the wide stages); wave 0 of a consumer polls the counter (bounded; a wait that
-// runs out, or sees another's failure, stops the workgroup's walk and sets the sticky
-// error word), then the workgroup reads with plain loads.  Every dependency points
-// back and every workgroup is resident, so every wait ends.  The last workgroup out
-// resets the counters and ORs a failure into the status word.
-constexpr int FP_LINE = 32, FP_LANES = 16;
+// drain, pass a barrier and add to every copy of the counter (FP_WIDE); wave 0 of a
+// consumer polls one copy (bounded; a wait that runs out, or sees another's failure,
+// stops the workgroup's walk and sets the sticky error word), then the workgroup reads with
+// plain loads.  Every dependency points back and every workgroup is resident, so every
+// wait ends.  The last workgroup out resets the counters and ORs a failure into the
+// status word.
+constexpr int FP_LINE = 32;
+// Device-coherent accesses to one line are served one after another, about 15 ns each, so
+// 256 workgroups polling the same counter lines come back every 4 us.  A counter is split
+// into FP_LANES sub-counters for its producers, and kept FP_COPIES times for its
+// consumers: a producer's one instruction adds to every copy, a workgroup polls copy
+// blockIdx % FP_COPIES.  32 rows of the FP8 front: 40.4 -> 37.7 us (8 x 4; 4 x 8, 16 x 8
+// and 4 x 16 the same).  Not so in the layer's stages, whose waits other work hides: the
+// same copies there gave nothing, and their reset (one store a line) cost 1.2 us.
+constexpr int FP_LANES = 8, FP_COPIES = 4, FP_WIDE = FP_LANES * FP_COPIES;
 // the front shapes the front-and-layer launch instantiates (with A8W4 experts): C7's
 // GEMV steps and nope 192, block-FP8 weights row-major or in AITER's layout
 enum : int { FRONT_FUSED_NONE = 0, FRONT_FUSED_C7_FP8 = 1, FRONT_FUSED_C7_AITER16 = 2 };
 enum : int {
-  FP_NORM = 0,                 // normed rows done
-  FP_A = 1,                    // [FP_LANES] hidden-input GEMV workgroups done
-  FP_ROWS = FP_A + FP_LANES,   // [FP_LANES] per-row tasks done
-  FP_C = FP_ROWS + FP_LANES,   // [FP_LANES] q_an-input GEMV workgroups done
-  FP_DONE = FP_C + FP_LANES,   // workgroups finished
+  FP_DONE = 49,                // workgroups finished
   FP_ERR,                      // sticky within a launch
   FP_STATUS,                   // nonzero once a launch failed; never cleared here
-  FP_HEADS,                    // [FP_LANES] per-head tasks done (when the layer follows in the launch)
-  FP_LINES = FP_HEADS + FP_LANES
+  // wide counters, [FP_WIDE] each
+  FP_NORM = 64,                // normed rows done
+  FP_A = FP_NORM + FP_WIDE,    // hidden-input GEMV workgroups done
+  FP_ROWS = FP_A + FP_WIDE,    // per-row tasks done
+  FP_C = FP_ROWS + FP_WIDE,    // q_an-input GEMV workgroups done
+  FP_HEADS = FP_C + FP_WIDE,   // per-head tasks done (when the layer follows in the launch)
+  FP_LINES = FP_HEADS + FP_WIDE
 };
 static_assert(FP_STATUS * FP_LINE * 4 == MK2_FRONT_STATUS_OFFSET, "the status word's documented offset");
 
@@ -567,23 +576,26 @@ union FrontLds {
 
 MK2_DEV int* fp_ctr(const FrontPDev& p, int line) { return p.sync + line * FP_LINE; }
 
-MK2_DEV void fp_signal(const FrontPDev& p, int line, int t, int lanes) {
+// producer t's task onto every copy of a wide counter (one instruction)
+MK2_DEV void fp_signal(const FrontPDev& p, int line, int t) {
   drain_memory();
   __syncthreads();
-  if (threadIdx.x == 0)
-    __hip_atomic_fetch_add(fp_ctr(p, line + t % lanes), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x < FP_COPIES)
+    __hip_atomic_fetch_add(fp_ctr(p, line + threadIdx.x * FP_LANES + t % FP_LANES), 1, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// until the sub-counters of `line` sum to target; seen[k] (k < FP_SEEN - 1) caches what
-// wait k saw and seen[FP_SEEN - 1] is the workgroup's failure flag (every thread
-// returns the same)
+// until the sub-counters of this workgroup's copy of `line` sum to target; seen[k] (k <
+// FP_SEEN - 1) caches what wait k saw and seen[FP_SEEN - 1] is the workgroup's failure
+// flag (every thread returns the same)
 constexpr int FP_SEEN = 8;
-MK2_DEV bool fp_wait(const FrontPDev& p, int* seen, int k, int line, int lanes, int target) {
+MK2_DEV bool fp_wait(const FrontPDev& p, int* seen, int k, int line, int target) {
+  constexpr int lanes = FP_LANES;
   if (seen[k] >= target) return true;
   int v = 0;
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
-    const int* ctr = fp_ctr(p, line + min(lane, lanes - 1));
+    const int* ctr = fp_ctr(p, line + blockIdx.x % FP_COPIES * FP_LANES + min(lane, lanes - 1));
     const int* err = fp_ctr(p, FP_ERR);
     auto poll = [&]() { return __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     auto count = [&](int c) { return __builtin_amdgcn_readfirstlane(row16_sum_i32(lane < lanes ? c : 0)); };
@@ -632,41 +644,41 @@ MK2_DEV bool front_walk(const FrontPDev& p, FrontLds& S, int* seen) {
   // 0. the normed input rows
   FP_TASKS(t, M) {
     front_norm_row(p.x, p.g_in, p.x_n, p.hidden, p.eps, t, S.rows.sh);
-    fp_signal(p, FP_NORM, 0, 1);
+    fp_signal(p, FP_NORM, t);
   }
   FP_NEXT(M);
   // 1. the hidden-input GEMVs, per pass: [W_qkv_a | W_ik], then W_iw
   const int nA = p.gridA + p.gridW;
   FP_TASKS(t, p.passes * nA) {
     const int pass = t / nA, u = t % nA;
-    auto w = [&] { return fp_wait(p, seen, 0, FP_NORM, 1, M); };
+    auto w = [&] { return fp_wait(p, seen, 0, FP_NORM, M); };
     const bool ok = u < p.gridA ? gemv_run<KUA, WF, NCG>(p.A[pass], u, p.gridA, S.gemv, w)
                                 : gemv_run<1, MK2_WFMT_BF16, NCG>(p.W[pass], u - p.gridA, p.gridW, S.gemv, w);
     if (!ok) return false;
-    fp_signal(p, FP_A, t, FP_LANES);
+    fp_signal(p, FP_A, t);
   }
   FP_NEXT(p.passes * nA);
   // 2. the per-row stage
   const int nR = (p.f.ih ? 3 : 2) * M;
   FP_TASKS(t, nR) {
-    if (!fp_wait(p, seen, 1, FP_A, FP_LANES, p.passes * nA)) return false;
+    if (!fp_wait(p, seen, 1, FP_A, p.passes * nA)) return false;
     front_rows_task(p.f, t, S.rows.sh, S.rows.kvv);
-    fp_signal(p, FP_ROWS, t, FP_LANES);
+    fp_signal(p, FP_ROWS, t);
   }
   FP_NEXT(nR);
   // 3. the q_an-input GEMVs
   FP_TASKS(t, p.passes * p.gridC) {
     const int pass = t / p.gridC, u = t % p.gridC;
-    if (!gemv_run<KUC, WF, NCG>(p.C[pass], u, p.gridC, S.gemv, [&] { return fp_wait(p, seen, 2, FP_ROWS, FP_LANES, nR); }))
+    if (!gemv_run<KUC, WF, NCG>(p.C[pass], u, p.gridC, S.gemv, [&] { return fp_wait(p, seen, 2, FP_ROWS, nR); }))
       return false;
-    fp_signal(p, FP_C, t, FP_LANES);
+    fp_signal(p, FP_C, t);
   }
   FP_NEXT(p.passes * p.gridC);
   // 4. the per-head stage
   FP_TASKS(t, p.nheads) {
-    if (!front_heads_task<NS>(p.f, t, S.qn, [&] { return fp_wait(p, seen, 3, FP_C, FP_LANES, p.passes * p.gridC); }))
+    if (!front_heads_task<NS>(p.f, t, S.qn, [&] { return fp_wait(p, seen, 3, FP_C, p.passes * p.gridC); }))
       return false;
-    if constexpr (HEADS) fp_signal(p, FP_HEADS, t, FP_LANES);
+    if constexpr (HEADS) fp_signal(p, FP_HEADS, t);
     else __syncthreads();  // this workgroup's next head task rewrites qn
   }
 #undef FP_TASKS
@@ -679,7 +691,7 @@ MK2_DEV bool front_walk(const FrontPDev& p, FrontLds& S, int* seen) {
 MK2_DEV void front_reset(const FrontPDev& p) {
   if (threadIdx.x == 0 && __hip_atomic_load(fp_ctr(p, FP_ERR), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
     atomicOr(fp_ctr(p, FP_STATUS), 1);
-  for (int l = threadIdx.x; l < FP_LINES; l += FR_NT)
+  for (int l = FP_DONE + (int)threadIdx.x; l < FP_LINES; l += FR_NT)
     if (l != FP_STATUS) __hip_atomic_store(fp_ctr(p, l), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 

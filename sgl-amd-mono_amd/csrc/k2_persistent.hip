@@ -271,7 +271,7 @@ struct K2Front {
   FrontPDev f;
   MK2_DEV bool run(FrontLds& S, int* seen) const {
     if (!front_walk<KUA, KUC, WF, NS, NCG, true>(f, S, seen)) return false;
-    return fp_wait(f, seen, 4, FP_HEADS, FP_LANES, f.nheads);
+    return fp_wait(f, seen, 4, FP_HEADS, f.nheads);
   }
   MK2_DEV void reset() const { front_reset(f); }
 };

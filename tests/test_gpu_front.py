@@ -307,3 +307,20 @@ def test_front_above_16_rows_matches_narrow_calls(wfmt, hidden, q_lora, heads, i
 
     for x, y in zip(run([(0, rows)]), run([(0, 16), (16, rows)])):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("rows", [1, 7, 9, 31])
+def test_front_counter_copies(rows):
+    """Fewer tasks than a counter's sub-counters, one more, and the most: the persistent
+    front gives the staged launches' bits, launch after launch."""
+    from sgl_amd_mono.k2 import config as C
+    from sgl_amd_mono.k2 import synth
+
+    dev = _dev()
+    ns = synth.make_front(C.C7_FRONT, rows, 640 + rows, dev)
+    op, res = _front_outputs(C.C7_FRONT, ns, rows, staged=False, repeats=4)
+    _, ref = _front_outputs(C.C7_FRONT, ns, rows, staged=True)
+    assert op.persistent and op.status() == 0
+    for launch in res:
+        for a, b in zip(launch, ref[0]):
+            assert torch.equal(a, b)
