@@ -117,17 +117,12 @@ __global__ __launch_bounds__(FR_NT, 1) void k_front_persistent(FrontPDev p) {
   __shared__ FrontLds S;
   __shared__ int seen[FP_SEEN];
   __shared__ int last;
-  const int G = gridDim.x;
   if (threadIdx.x < FP_SEEN) seen[threadIdx.x] = 0;
   __syncthreads();
   front_walk<KUA, KUC, WF, NS, NCG>(p, S, seen);
   // the last workgroup out resets the counters for the next launch
-  drain_memory();
-  __syncthreads();
-  if (threadIdx.x == 0)
-    last = __hip_atomic_fetch_add(fp_ctr(p, FP_DONE), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == G - 1;
-  __syncthreads();
-  if (last) front_reset(p);
+  bool failed;
+  if (launch_exit(fp_ctr(p, FP_EXIT), gridDim.x, &last, &failed)) front_reset(p, failed);
 }
 
 static int front_cus() {

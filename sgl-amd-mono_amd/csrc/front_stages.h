@@ -522,7 +522,7 @@ MK2_DEV bool front_heads_task(const FrontDev& p, int b, uint4* qn, Wait wait = W
 // persistent layer does: producers store their hand-off data device-coherently,
 // drain, pass a barrier and add to every copy of the counter (FP_WIDE); wave 0 of a
 // consumer polls one copy (bounded; a wait that runs out, or sees another's failure,
-// stops the workgroup's walk and sets the sticky error word), then the workgroup reads with
+// stops the workgroup's walk and marks the launch failed), then the workgroup reads with
 // plain loads.  Every dependency points back and every workgroup is resident, so every
 // wait ends.  The last workgroup out resets the counters and ORs a failure into the
 // status word.
@@ -539,8 +539,7 @@ constexpr int FP_LANES = 8, FP_COPIES = 4, FP_WIDE = FP_LANES * FP_COPIES;
 // GEMV steps and nope 192, block-FP8 weights row-major or in AITER's layout
 enum : int { FRONT_FUSED_NONE = 0, FRONT_FUSED_C7_FP8 = 1, FRONT_FUSED_C7_AITER16 = 2 };
 enum : int {
-  FP_DONE = 49,                // workgroups finished
-  FP_ERR,                      // sticky within a launch
+  FP_EXIT = 50,                // workgroups finished, and a failed wait (launch_exit)
   FP_STATUS,                   // nonzero once a launch failed; never cleared here
   // wide counters, [FP_WIDE] each
   FP_NORM = 64,                // normed rows done
@@ -596,7 +595,7 @@ MK2_DEV bool fp_wait(const FrontPDev& p, int* seen, int k, int line, int target)
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
     const int* ctr = fp_ctr(p, line + blockIdx.x % FP_COPIES * FP_LANES + min(lane, lanes - 1));
-    const int* err = fp_ctr(p, FP_ERR);
+    const int* err = fp_ctr(p, FP_EXIT);
     auto poll = [&]() { return __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     auto count = [&](int c) { return __builtin_amdgcn_readfirstlane(row16_sum_i32(lane < lanes ? c : 0)); };
     bool bad = false;
@@ -610,12 +609,12 @@ MK2_DEV bool fp_wait(const FrontPDev& p, int* seen, int k, int line, int target)
       v = count(c1);
       if (v >= target) break;
       n += 2;
-      if ((n & 31) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+      if ((n & 31) == 0 && launch_failing(err)) {
         bad = true;
         break;
       }
       if (wc.expired(p.wait_ticks)) {
-        if (lane == 0) atomicOr(fp_ctr(p, FP_ERR), 1);
+        if (lane == 0) launch_fail(fp_ctr(p, FP_EXIT));
         bad = true;
         break;
       }
@@ -686,12 +685,11 @@ MK2_DEV bool front_walk(const FrontPDev& p, FrontLds& S, int* seen) {
   return true;
 }
 
-// the last workgroup out (every workgroup counted out on FP_DONE): a failure into the
-// status word, every counter back to zero for the next launch
-MK2_DEV void front_reset(const FrontPDev& p) {
-  if (threadIdx.x == 0 && __hip_atomic_load(fp_ctr(p, FP_ERR), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-    atomicOr(fp_ctr(p, FP_STATUS), 1);
-  for (int l = FP_DONE + (int)threadIdx.x; l < FP_LINES; l += FR_NT)
+// the last workgroup out: a failure of the front's own (the launch `failed`) into the status
+// word, every counter back to zero for the next launch
+MK2_DEV void front_reset(const FrontPDev& p, bool failed) {
+  if (failed && threadIdx.x == 0 && launch_failing(fp_ctr(p, FP_EXIT))) atomicOr(fp_ctr(p, FP_STATUS), 1);
+  for (int l = FP_EXIT + (int)threadIdx.x; l < FP_LINES; l += FR_NT)
     if (l != FP_STATUS) __hip_atomic_store(fp_ctr(p, l), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 

@@ -655,8 +655,8 @@ MK2_DEV bool idx_slice(const IdxDev& p, int r, int chunk, TopkLds& S, uint32_t w
       for (int polls = 1;; ++polls) {
         v = lane < chunk ? ld_dev_i32(cc + lane) : CC_FLAG;
         if (__ballot((v & CC_FLAG) == 0) == 0) break;
-        if (wc.expired(wait_ticks) || ((polls & 31) == 0 && err && ld_dev_i32(err))) {
-          if (lane == 0 && err) atomicOr(err, 1);
+        if (wc.expired(wait_ticks) || ((polls & 31) == 0 && err && launch_failing(err))) {
+          if (lane == 0 && err) launch_fail(err);
           break;
         }
       }

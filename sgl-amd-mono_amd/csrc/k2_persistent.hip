@@ -40,8 +40,7 @@ enum : int {
   SY_UPW = 80,     // [K2_LANES] workgroups through the up/gate tasks (above 16 rows)
   SY_SPLIT = 96,   // [32] attention splits done, per row
   SY_ROUTE = 128,  // the routing's table and list are out (the down)
-  SY_DONE = 130,   // workgroups finished (the last one resets)
-  SY_ERR,          // sticky: a wait passed its deadline
+  SY_EXIT = 130,   // workgroups finished (the last one resets), and a failed wait (launch_exit)
   SY_UV = 144,     // [K2_LANES] sub-counters each: merged + W_UV (row group, head, half) tasks
   SY_OPROJ = SY_UV + K2_LANES,
   SY_ROUTER = SY_OPROJ + K2_LANES,
@@ -114,6 +113,13 @@ MK2_DEV void k2_count(const K2Dev& p, int line) {
   __hip_atomic_fetch_add(k2_ctr(p, line), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// the last workgroup out: lines [l0, l1) and the exit word back to zero
+MK2_DEV void k2_reset(const K2Dev& p, int l0, int l1) {
+  for (int l = l0 + (int)threadIdx.x; l < l1; l += K2_NT)
+    __hip_atomic_store(k2_ctr(p, l), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) __hip_atomic_store(k2_ctr(p, SY_EXIT), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // publish n finished tasks on counter `line` (sub-counter t mod lanes): every thread's
 // stores drained, then one increment
 MK2_DEV void k2_signal(const K2Dev& p, int line, int t = 0, int lanes = 1, int n = 1) {
@@ -146,7 +152,7 @@ MK2_DEV bool k2_wait(const K2Dev& p, int* seen, int line, int target, int stamp 
   bool bad = false;
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
-    const int* err = k2_ctr(p, SY_ERR);
+    const int* err = k2_ctr(p, SY_EXIT);
     const int* ctr = k2_ctr(p, line + min(lane, lanes - 1));
     // two polls in flight: the next is issued before the last one's count is read
     auto poll = [&]() { return __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
@@ -163,12 +169,12 @@ MK2_DEV bool k2_wait(const K2Dev& p, int* seen, int line, int target, int stamp 
       v = count(c1);
       if (v >= target) break;
       n += 2;
-      if ((n & 31) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+      if ((n & 31) == 0 && launch_failing(err)) {
         bad = true;
         break;
       }
       if (wc.expired(p.wait_ticks)) {
-        if (lane == 0) atomicOr(k2_ctr(p, SY_ERR), 1);
+        if (lane == 0) launch_fail(k2_ctr(p, SY_EXIT));
         bad = true;
         break;
       }
@@ -264,7 +270,7 @@ constexpr int K2_KEEP = 4;
 // counters.
 struct K2NoFront {
   MK2_DEV bool run(FrontLds&, int*) const { return true; }
-  MK2_DEV void reset() const {}
+  MK2_DEV void reset(bool) const {}
 };
 template <int KUA, int KUC, int WF, int NS, int NCG>
 struct K2Front {
@@ -273,7 +279,7 @@ struct K2Front {
     if (!front_walk<KUA, KUC, WF, NS, NCG, true>(f, S, seen)) return false;
     return fp_wait(f, seen, 4, FP_HEADS, f.nheads);
   }
-  MK2_DEV void reset() const { front_reset(f); }
+  MK2_DEV void reset(bool failed) const { front_reset(f, failed); }
 };
 
 template <int NCG, int FMT, class Front = K2NoFront>
@@ -296,7 +302,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
   if (threadIdx.x == 0) epoch = (uint32_t)ld_dev_i32(p.sync + SYNC_EPOCH);
   auto tag_of = [](uint32_t e) { return e + 1u ? e + 1u : 1u; };
   __syncthreads();
-  TagPoll tp{0u, p.wait_ticks, k2_ctr(p, SY_ERR)};
+  TagPoll tp{0u, p.wait_ticks, k2_ctr(p, SY_EXIT)};
   // the stages in order; a wait that fails (its deadline, or another workgroup's
   // failure seen while polling) returns from the walk: the workgroup skips every task
   // left and goes straight to the counter reset (fail-stop)
@@ -338,7 +344,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
       const int r = t / nchk;
       if (!k2_wait(*pp, seen, SY_SCORE + r, nchk, t < G ? 3 * st + 1 : -1)) return;
       bool last = false;
-      const bool known = idx_slice<K2_NT>(pp->idx, r, t % nchk, S.topk, pp->wait_ticks, k2_ctr(*pp, SY_ERR), tp.tag,
+      const bool known = idx_slice<K2_NT>(pp->idx, r, t % nchk, S.topk, pp->wait_ticks, k2_ctr(*pp, SY_EXIT), tp.tag,
                                           [&] {
                                             if (sel_tasks)
                                               k2_signal(*pp, SY_SLICE + r);
@@ -499,7 +505,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
     __syncthreads();
     front_ok = front.run(S.front, fseen);
     __syncthreads();  // the front's LDS is the stages' from here on
-    if (!front_ok && threadIdx.x == 0) atomicOr(k2_ctr(p, SY_ERR), 1);
+    if (!front_ok && threadIdx.x == 0) launch_fail(k2_ctr(p, SY_EXIT));
   }
   if (front_ok) walk();
 #undef K2_TASKS
@@ -508,16 +514,9 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
   if (p.timeline && threadIdx.x < K2_STAMPS)
     p.timeline[(size_t)blockIdx.x * K2_STAMPS + threadIdx.x] = k2_lds_stamps[threadIdx.x];
   // ---- the last workgroup out resets the counters for the next launch
-  drain_memory();  // this workgroup's stores and atomics have landed before it counts out
-  __syncthreads();
-  if (threadIdx.x == 0)
-    last_flag = __hip_atomic_fetch_add(k2_ctr(p, SY_DONE), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == G - 1;
-  __syncthreads();
-  if (last_flag) {
-    __syncthreads();
-    if (threadIdx.x == 0) last_flag = __hip_atomic_load(k2_ctr(p, SY_ERR), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (last_flag) {
+  bool failed;
+  if (launch_exit(k2_ctr(p, SY_EXIT), G, &last_flag, &failed)) {
+    if (failed) {
       // a stopped launch skipped some rows' top-k resets: every workgroup has left, so
       // clear all rows' top-k state here and the next launch starts clean
       idx_reset_rows<K2_NT>(p.idx, R);
@@ -527,9 +526,8 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
     } else {  // the chunk counts (the selects cleared the histograms)
       for (int i = threadIdx.x; i < R * p.idx.nchk; i += K2_NT) st_dev_i32(p.idx.ccount + i, 0);
     }
-    for (int l = threadIdx.x; l < SY_LINES; l += K2_NT)
-      __hip_atomic_store(k2_ctr(p, l), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    front.reset();
+    k2_reset(p, 0, SY_LINES);
+    front.reset(failed);
     // the epoch moves on: the next launch's tags differ from every tag of this one
     if (threadIdx.x == 0) st_dev_i32(p.sync + SYNC_EPOCH, (int)tag_of(epoch));
   }
@@ -589,7 +587,7 @@ int k2_persistent_enqueue(const IdxDev& idx, const MlaDev& mla, const MoeDev& mo
 
 // ------------------------------------------------------------------------------------
 // The layer's three blocks as persistent launches of their own (the entry points of
-// configs[0..3]): the same stage functions, counters, hand-offs and fail-stop as the
+// the indexer, the sparse MLA and the MoE): the same stage functions, counters, hand-offs and fail-stop as the
 // layer's launch, walking only the block's stages.  The block's sync block leads its
 // workspace (zero-filled before the first launch; every launch leaves it so); a launch
 // whose wait gave up ORs 1 into the status word at BLOCK_STATUS_INT of it.
@@ -614,7 +612,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_block(K2Dev p) {
     s_tag = e ? e : 1u;
   }
   __syncthreads();
-  const TagPoll tp{s_tag, p.wait_ticks, k2_ctr(p, SY_ERR)};
+  const TagPoll tp{s_tag, p.wait_ticks, k2_ctr(p, SY_EXIT)};
   uint32_t sel_rows = 0;  // the rows whose select this workgroup ran
   auto walk = [&]() {
     // a new view a stage; one for the whole walk in the W8A8 MoE block, which ran 4 % slower
@@ -640,7 +638,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_block(K2Dev p) {
         const int r = t / nchk;
         if (!k2_wait(*pp, seen, SY_SCORE + r, nchk)) return;
         bool last = false;
-        const bool known = idx_slice<K2_NT>(pp->idx, r, t % nchk, S.topk, pp->wait_ticks, k2_ctr(*pp, SY_ERR), tp.tag,
+        const bool known = idx_slice<K2_NT>(pp->idx, r, t % nchk, S.topk, pp->wait_ticks, k2_ctr(*pp, SY_EXIT), tp.tag,
                                             [&] {
                                               if (sel_tasks)
                                                 k2_signal(*pp, SY_SLICE + r);
@@ -745,16 +743,9 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_block(K2Dev p) {
   };
   walk();
   // the last workgroup out resets the counters (and on a stop the top-k state it left)
-  drain_memory();
-  __syncthreads();
-  if (threadIdx.x == 0)
-    last_flag = __hip_atomic_fetch_add(k2_ctr(p, SY_DONE), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == G - 1;
-  __syncthreads();
-  if (last_flag) {
-    __syncthreads();
-    if (threadIdx.x == 0) last_flag = __hip_atomic_load(k2_ctr(p, SY_ERR), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (last_flag) {
+  bool failed;
+  if (launch_exit(k2_ctr(p, SY_EXIT), G, &last_flag, &failed)) {
+    if (failed) {
       if constexpr (BLK == K2_BLOCK_INDEXER) idx_reset_rows<K2_NT>(p.idx, R);
       if (threadIdx.x == 0) atomicOr(p.sync + BLOCK_STATUS_INT, 1);
       drain_memory();
@@ -762,8 +753,9 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_block(K2Dev p) {
     } else if constexpr (BLK == K2_BLOCK_INDEXER) {
       for (int i = threadIdx.x; i < R * p.idx.nchk; i += K2_NT) st_dev_i32(p.idx.ccount + i, 0);
     }
-    for (int l = threadIdx.x; l < SY_LINES; l += K2_NT)
-      __hip_atomic_store(k2_ctr(p, l), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (BLK == K2_BLOCK_INDEXER) k2_reset(p, SY_SCORE, SY_SLICE + R);
+    if constexpr (BLK == K2_BLOCK_MLA) k2_reset(p, SY_SPLIT, SY_UV + K2_LANES);
+    if constexpr (BLK == K2_BLOCK_MOE) k2_reset(p, SY_UPT, SY_LINES);
     if (threadIdx.x == 0) st_dev_i32(p.sync + SYNC_EPOCH, (int)s_tag);
   }
 }

@@ -86,3 +86,31 @@ def test_layer_step_refusals():
     step = LayerStepOp(FrontOp(bf, fb, rows, device=dev), LayerOp(C.C5_LAYER, L, rows, device=dev))
     with pytest.raises(_lib.Mk2Error, match="no instance"):
         step(positions, slots, fb.rope_cos_sin)
+
+
+@pytest.mark.parametrize("rows", [1, 8, 32])
+def test_layer_step_stop_and_next_launch(rows):
+    """A wait that gives up (deadline 1 us) marks the front-and-layer launch's exit word: the
+    front's and the layer's status words are set, and the launches after it, on the same
+    workspaces, give the bits of a first launch."""
+    from sgl_amd_mono.k2 import config as C
+    from sgl_amd_mono.k2 import synth
+    from sgl_amd_mono.k2.ops import FrontOp, LayerOp, LayerStepOp
+
+    dev = _dev()
+    fc = C.C7_FRONT
+    fw = synth.make_front(fc, rows, 930 + rows, dev)
+    L = synth.make_layer(C.C5_LAYER, rows, 940 + rows, dev)
+    positions, slots = _step_inputs(L, rows, 945 + rows, dev, fc.max_position)
+    fop, lop = FrontOp(fc, fw, rows, device=dev), LayerOp(C.C5_LAYER, L, rows, device=dev)
+    step = LayerStepOp(fop, lop)
+    ref = cpu(step(positions, slots, fw.rope_cos_sin))
+    lop.wait_us = 1
+    step(positions, slots, fw.rope_cos_sin)
+    assert int(lop.status.item()) == 1 and fop.status() == 1
+    lop.wait_us = 0
+    lop.status.zero_()
+    fop.status_word().zero_()
+    for _ in range(2):
+        assert torch.equal(cpu(step(positions, slots, fw.rope_cos_sin)), ref)
+    assert int(lop.status.item()) == 0 and fop.status() == 0
