@@ -602,13 +602,10 @@ MK2_DEV bool fp_wait(const FrontPDev& p, int* seen, int k, int line, int target)
     int n = 0, c0 = poll();
     WaitClock wc;
     while (true) {
-      const int c1 = poll();
       v = count(c0);
       if (v >= target) break;
       c0 = poll();
-      v = count(c1);
-      if (v >= target) break;
-      n += 2;
+      ++n;
       if ((n & 31) == 0 && launch_failing(err)) {
         bad = true;
         break;
