@@ -579,7 +579,7 @@ MK2_DEV void idx_clear_hist(const IdxDev& p, int r) {
 // while the slices still list their keys above the bin); then the task waits for the
 // earlier chunks' counts (tasks only wait on chunks of lower index, which publish
 // before they wait, so with every task started every wait ends; a wait past its
-// deadline of `wait_ticks` (WaitClock), or the sticky error word `err` set, gives up
+// deadline of `wait_ticks` (WaitClock), or the launch's exit word `err` marked failed, gives up
 // and sets it).  `kept`: the
 // chunk's scores in LDS (its score task's `keep`), or null: read from `scores`.
 // Returns whether S.res[0..1] now hold b1 and the count above it.

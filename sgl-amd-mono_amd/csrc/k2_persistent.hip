@@ -15,7 +15,7 @@
 // consumer polls the counter, passes a barrier and reads.  Dependencies point only
 // to earlier stages and every workgroup is resident (one per CU, grid = CU count),
 // so every wait ends; each wait is also bounded (a deadline) and on expiry sets a
-// sticky error word that releases every other wait, so the launch always drains.
+// failed bit of the exit word, which releases every other wait, so the launch always drains.
 // The last workgroup to finish resets the counters.
 #include "front_stages.h"
 #include "indexer_stages.h"
@@ -54,7 +54,7 @@ struct K2Dev {
   MlaDev mla;
   MoeDev moe;
   int* sync;
-  int* status;    // optional: the launch's error word
+  int* status;    // optional: set once a launch failed
   uint64_t* timeline;  // optional: [grid][K2_STAMPS] s_memrealtime stamps (100 MHz)
   int rows;
   uint32_t wait_ticks;  // a dependency wait's deadline (WaitClock ticks)
@@ -141,7 +141,7 @@ MK2_DEV bool k2_signal_last1(const K2Dev& p, int line, int n, int* flag) {
 }
 
 // wait until counter `line` (summed over `lanes` sub-counters) reaches `target`.  Wave
-// 0 polls, one coherent load a lane a poll; the error word every 32 polls.  `seen`
+// 0 polls, one coherent load a lane a poll; the exit word every 32 polls.  `seen`
 // (LDS, by line) caches the counts this workgroup has observed (counters only grow
 // within a launch), so a wait that an earlier one already satisfied costs nothing.  The
 // early return is uniform: seen is written only just after this function's barrier,
