@@ -375,7 +375,7 @@ MK2_DEV bool launch_failing(const int* word) { return (ld_dev_i32(word) & EXIT_F
 // one, which may reset the launch's counters, with *failed whether any wait gave up.
 // `lds`: one int.  (The failure in a word of its own cost the last workgroup one more round
 // trip after every other had left.  With it and a reset of only the lines the launch uses,
-// 0.3 to 0.5 us a launch: the indexer's at 1 x 2048 19.75 -> 19.4, at 8 x 65536 23.2 -> 22.7.)
+// 0.3 to 0.5 us a launch: the indexer's at 1 x 4096 19.75 -> 19.4, at 8 x 65536 23.2 -> 22.7.)
 MK2_DEV bool launch_exit(int* word, int G, int* lds, bool* failed) {
   drain_memory();
   __syncthreads();
