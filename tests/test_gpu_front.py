@@ -216,7 +216,7 @@ def test_front_persistent_matches_staged(case):
     """The persistent front (one launch, counters between its stages) gives the six
     stage launches' bits -- outputs, latent and index cache rows and scales -- on
     back-to-back launches (its counters reset by the launch itself), at 1, 8 and 32
-    rows (two GEMV passes), bf16 weights, AITER's layout, hidden 7168 without the
+    rows, bf16 weights, AITER's layout, hidden 7168 without the
     indexer; its status word stays 0."""
     from sgl_amd_mono.k2 import config as C
     from sgl_amd_mono.k2 import synth
