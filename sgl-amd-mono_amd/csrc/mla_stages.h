@@ -11,6 +11,7 @@
 // oproj task (16 hidden rows): a = bf16(h + W_o o) on bf16 MFMA.
 #pragma once
 #include "mk2_device.h"
+#include "mla_table.h"
 
 namespace mk2 {
 
@@ -123,11 +124,8 @@ MK2_DEV bool mla_split_tasks(const MlaDev& p, int t0, int t1, int iters, MlaSpli
     return (int)pair_value(w);
   };
   // (the page's load has no use here to wait for)
-  auto on_page = [&](int pos) { return pos >= 0 && pos < p.stride * 64; };
-  auto page_of = [&](int t, int pos) {
-    return p.pt[(size_t)p.req[t / p.nsplit] * p.stride + (on_page(pos) ? pos >> 6 : 0)];
-  };
-  auto cache_row = [&](int pos, int page) { return on_page(pos) ? page * 64 + (pos & 63) : -1; };
+  auto page_of = [&](int t, int pos) { return mla_page(p.pt, p.req, t / p.nsplit, p.stride, pos); };
+  auto cache_row = [&](int pos, int page) { return mla_cache_row(pos, page, p.stride); };
   // gather: 16-byte piece i % 36 of key i / 36; every load of a thread is issued at once,
   // the rows' scales ahead of them
   constexpr int PIECES = MLA_SPLIT * (MLA_D / 16), PPT = (PIECES + NT - 1) / NT;
