@@ -94,14 +94,17 @@ union K2Lds {
 static_assert(sizeof(FrontLds) <= sizeof(TopkLds), "the front's LDS fits the layer's union as it is");
 
 // The launch's K2Dev (each kernel's first argument) as its kernel-argument memory, behind a
-// pointer the compiler cannot see through: a stage that takes it anew loads the pointers
-// and sizes it uses as it starts (scalar cache hits).  With one view of the arguments for
-// the whole walk they were loaded up front and lived, spilled to vector lanes, through
-// every stage: 205 of them at 32 rows and 264 at 8 of the A8W4 layer, now 96 and 116 (vector
-// spills at 32 rows 38 -> 24), and the layer 225.7 -> 214.4 us at 32 rows, the indexer's
-// launch 23.4 -> 22.9 at 8 x 65536.
-MK2_DEV const K2Dev* k2_args() {
-  auto a = (const __attribute__((address_space(4))) K2Dev*)__builtin_amdgcn_kernarg_segment_ptr();
+// pointer the compiler cannot see through: a stage that takes a new view of it loads the
+// pointers and sizes it uses as it starts (scalar cache hits).  With one view of the
+// arguments for the whole walk they were loaded up front and lived, spilled to vector lanes,
+// through every stage: 205 of them at 32 rows and 264 at 8 of the A8W4 layer, with a view a
+// stage 96 and 116 (vector spills at 32 rows 38 -> 24), and the layer 225.7 -> 214.4 us at
+// 32 rows, the indexer's launch 23.4 -> 22.9 at 8 x 65536.
+// A kernel takes the pointer in its own body, K2_ARGS: in a function that is not inlined
+// into it the builtin is 0.
+using K2Args = const __attribute__((address_space(4))) K2Dev*;
+#define K2_ARGS ((K2Args)__builtin_amdgcn_kernarg_segment_ptr())
+MK2_DEV const K2Dev* k2_view(K2Args a) {
   asm volatile("" : "+s"(a));
   return (const K2Dev*)a;
 }
@@ -284,6 +287,7 @@ struct K2Front {
 
 template <int NCG, int FMT, class Front = K2NoFront>
 __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
+  const K2Args args = K2_ARGS;
   __shared__ K2Lds S;
   __shared__ float kept[K2_KEEP][IDX_CHUNK];  // this workgroup's score tasks' scores, by t / G
   __shared__ int seen[SY_LINES + 1];  // counts seen by line; [SY_LINES]: a wait failed
@@ -307,7 +311,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
   // failure seen while polling) returns from the walk: the workgroup skips every task
   // left and goes straight to the counter reset (fail-stop)
   auto walk = [&]() {
-    const K2Dev* pp = k2_args();
+    const K2Dev* pp = k2_view(args);
     int base = 0;  // this stage's first workgroup
     // the tasks of a stage of n tasks on this workgroup; `t < G` marks the first
 #define K2_TASKS(t, n) for (int t = (b - base % G + G) % G; t < (n); t += G)
@@ -325,7 +329,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
     if (threadIdx.x == 0) s_tag = tag_of(epoch);
     __syncthreads();
     tp.tag = s_tag;
-    pp = k2_args();
+    pp = k2_view(args);
     // ---- top-k slices: each chunk lists its keys above the row's threshold bin and
     // keeps its keys in the bin
     k2_stamp(*pp, 3 * st);
@@ -374,7 +378,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
       K2_NEXT(R);
     }
     st += 2;  // the select stamps are taken above
-    pp = k2_args();
+    pp = k2_view(args);
     // ---- sparse-MLA splits
     k2_stamp(*pp, 3 * st);
     const int ns = pp->mla.nsplit;
@@ -383,7 +387,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
     if (!k2_splits<NCG>(*pp, S, (b - base % G + G) % G, tp, [&](int) { k2_stamp(*pp, 3 * st + 1); })) return;
     K2_NEXT(R * ns);
     k2_stamp(*pp, 3 * st++ + 2);
-    pp = k2_args();
+    pp = k2_view(args);
     // ---- merge of the splits + W_UV, per (group of mrg rows, head, half of the head's
     // outputs): about one task a workgroup
     k2_stamp(*pp, 3 * st);
@@ -400,7 +404,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
     }
     K2_NEXT(nmt);
     k2_stamp(*pp, 3 * st++ + 2);
-    pp = k2_args();
+    pp = k2_view(args);
     // ---- W_o + residual, per 16 hidden rows: tasks t and t + G together (their weights
     // all in flight before the wait)
     k2_stamp(*pp, 3 * st);
@@ -414,7 +418,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
     }
     K2_NEXT(ht);
     k2_stamp(*pp, 3 * st++ + 2);
-    pp = k2_args();
+    pp = k2_view(args);
     // ---- router GEMV (+ RMSNorm of its slice), per (16 experts, hidden slice): the
     // partial logits go out as tagged words (the routing polls them); the counter
     // publishes the normalized rows the tasks of the first expert tile store
@@ -428,7 +432,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
     }
     K2_NEXT(nrt);
     k2_stamp(*pp, 3 * st++ + 2);
-    pp = k2_args();
+    pp = k2_view(args);
     // ---- routing, on one workgroup up to 8 rows: one without a router task (it polls
     // while they run) and with the fewest up/gate tasks.  It polls the router tasks' logits and
     // puts out the tagged expert list, then the route-weight table, published by
@@ -463,7 +467,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
       }
     }
     ++st;
-    pp = k2_args();
+    pp = k2_view(args);
     // ---- up/gate + SwiGLU: the shared expert's chunks first (they need only the
     // normalized rows, so they run while routing is still pending), then the routed
     // slots, each polling its slot of the tagged expert list
@@ -484,7 +488,7 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_layer(K2Dev p, Front front) {
     }
     K2_NEXT(up_total);
     k2_stamp(*pp, 3 * st++ + 2);
-    pp = k2_args();
+    pp = k2_view(args);
     // ---- down + route weighting + residual, per 16 hidden rows
     k2_stamp(*pp, 3 * st);
     K2_TASKS(t, down_tasks(pp->moe)) {
@@ -598,6 +602,7 @@ enum { K2_BLOCK_INDEXER = 0, K2_BLOCK_MLA = 1, K2_BLOCK_MOE = 2 };
 
 template <int BLK, int NCG, int FMT>
 __global__ __launch_bounds__(K2_NT, 1) void k_k2_block(K2Dev p) {
+  const K2Args args = K2_ARGS;
   __shared__ K2Lds S;
   __shared__ float kept[BLK == K2_BLOCK_INDEXER ? K2_KEEP : 1][IDX_CHUNK];
   __shared__ int seen[SY_LINES + 1];
@@ -618,8 +623,8 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_block(K2Dev p) {
     // a new view a stage; one for the whole walk in the W8A8 MoE block, which ran 4 % slower
     // with one a stage (117.5 -> 122.3 us at 13 rows)
     constexpr bool one_view = BLK == K2_BLOCK_MOE && FMT == MK2_FMT_W8A8;
-    const K2Dev* pp = one_view ? &p : k2_args();
-    auto next_view = [&] { if (!one_view) pp = k2_args(); };
+    const K2Dev* pp = one_view ? &p : k2_view(args);
+    auto next_view = [&] { if (!one_view) pp = k2_view(args); };
     int base = 0;
 #define K2_TASKS(t, n) for (int t = (b - base % G + G) % G; t < (n); t += G)
 #define K2_NEXT(n) base = (base + (n)) % G
