@@ -280,6 +280,32 @@ def test_persistent_layer_fail_stop():
     op.check()  # a clean launch: no error
 
 
+@pytest.mark.parametrize("rows", [17, 32])
+def test_persistent_layer_fail_stop_above_16_rows(rows):
+    """The same above 16 rows, where the splits run on half workgroups whose last wave polls
+    the list for the tasks after the current one and stops both halves."""
+    from sgl_amd_mono.k2 import config as C
+    from sgl_amd_mono.k2 import synth
+    from sgl_amd_mono.k2.ops import LayerOp
+
+    dev = _dev()
+    L = synth.make_layer(C.C5_LAYER, rows, 780 + rows, dev)
+    op = LayerOp(C.C5_LAYER, L, rows, device=dev)
+    ref = op().clone()
+    for _ in range(2):
+        op.wait_us = 1
+        op()
+        torch.cuda.synchronize()
+        assert int(op.status.item()) == 1
+        op.wait_us = 0
+        outs = [op().clone() for _ in range(2)]
+        with pytest.raises(RuntimeError, match="stopped early"):
+            op.check()
+        for o in outs:
+            assert torch.equal(o, ref)
+    op.check()
+
+
 @pytest.mark.parametrize("rows", [8, 32])
 def test_layer_aiter_layout_bits(rows):
     """The persistent layer with its experts in AITER's (16, 16) layout gives the
