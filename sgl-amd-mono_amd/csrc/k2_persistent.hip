@@ -620,9 +620,12 @@ __global__ __launch_bounds__(K2_NT, 1) void k_k2_block(K2Dev p) {
   const TagPoll tp{s_tag, p.wait_ticks, k2_ctr(p, SY_EXIT)};
   uint32_t sel_rows = 0;  // the rows whose select this workgroup ran
   auto walk = [&]() {
-    // a new view a stage; one for the whole walk in the W8A8 MoE block, which ran 4 % slower
-    // with one a stage (117.5 -> 122.3 us at 13 rows)
-    constexpr bool one_view = BLK == K2_BLOCK_MOE && FMT == MK2_FMT_W8A8;
+    // a new view a stage, but one for the whole walk in the W8A8 MoE block up to 16 rows,
+    // where it is the better one at most widths (hidden 6144, 256 experts of 256, one view
+    // against one a stage: 1 row 43.3 / 40.1 us, 4 rows 52.8 / 52.2, 8 rows 75.1 / 76.0, 13
+    // rows 98.7 / 100.3, 16 rows 107.2 / 108.4).  Above, one view is 3-5 % slower: 17 rows
+    // 141.9 / 135.5, 24 rows 166.0 / 159.5, 32 rows 189.2 / 183.0
+    constexpr bool one_view = BLK == K2_BLOCK_MOE && FMT == MK2_FMT_W8A8 && NCG == 1;
     const K2Dev* pp = one_view ? &p : k2_view(args);
     auto next_view = [&] { if (!one_view) pp = k2_view(args); };
     int base = 0;
