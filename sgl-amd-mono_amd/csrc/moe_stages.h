@@ -1276,50 +1276,84 @@ MK2_DEV void down_rows(const MoeDev& p, int nt, float* red, int* act_ids, float*
   // scaled MFMA against the E4M3 mid (W8A8, f32 scale per 128 a row), each k-block's product
   // times its scales and the route weight; or E2M1 weights widened exactly to bf16 against
   // the bf16 mid (A16W4), the slot's sum times the route weight.  DEPTH - 1 units are in
-  // flight while one computes, as many as the registers hold without spills.  Slot by slot
+  // flight while one computes, as many as the registers hold without spills up to 16 rows;
+  // above, the MoE block spills 8 (W8A16), 13 (W8A8) and 22 (A16W4) of them.  Slot by slot
   // (a slot's loads, then its products, in 16-row tasks) the block took 88.7 us at 8 rows of
   // hidden 6144 (256 experts of 256) in W8A16 and 67 in A16W4, now 71.1 and 47.8; W8A8 at 13
   // rows 117.6 -> 96.8
   constexpr bool w8a8 = FMT == MK2_FMT_W8A8, a16w4 = FMT == MK2_FMT_A16W4;
   constexpr int KCB = NCG == 1 || (w8a8 && DT == 1) ? 2 : 1;  // k-blocks a unit
   constexpr int DEPTH = w8a8 ? (DT == 1 && NCG == 1 ? 3 : 2) : NCG == 2 || a16w4 ? 3 : 2;
+  // W8A8's units of two k-blocks run on from a slot of the wave to its next.  With units of a
+  // slot's own, an odd number of k-blocks left each slot's last unit half empty, its block
+  // loaded twice (64 experts, hidden 2048: inter 384 at 17 rows 65.9 us, now 58.3, inter 896
+  // 122.6 and 111.0, inter 128 at 8 rows 33.9 and 31.6).  In W8A16 the same gained 2 us at
+  // odd numbers and lost 2-4 at even ones.
+  constexpr bool RUN_ON = w8a8 && KCB > 1;
+  constexpr int NSL = RUN_ON ? KCB : 1;  // slots a unit
   struct UnitB {
     uint4 a[DT][KCB][a16w4 ? 1 : 2];
     i32x8 bq[w8a8 ? KCB : 1][NCG];        // W8A8
     bf16x8 bb[w8a8 ? 1 : KCB][NCG][4];    // W8A16, A16W4
     float sc[DT][KCB];                    // E4M3: the block scales
     uint32_t sw[DT];                     // E2M1: the E8M0 words
-    float ms[w8a8 ? KCB : 1][NCG], wr[NCG];
+    float ms[w8a8 ? KCB : 1][NCG], wr[NSL][NCG];
   };
-  const int nkcb = (KB2 + KCB - 1) / KCB;  // units a slot
-  const int nub = !mx && D > wave ? (D - wave + NW - 1) / NW * nkcb : 0;
+  const int nsl = !mx && D > wave ? (D - wave + NW - 1) / NW : 0;  // the wave's slots
+  const int nkcb = (KB2 + KCB - 1) / KCB;                          // units a slot (not RUN_ON)
+  const int nub = RUN_ON ? (nsl * KB2 + KCB - 1) / KCB : nsl * nkcb;
+  // unit u's slots and k-blocks (past the end a valid one, unused)
+  struct Blocks {
+    int j[NSL], kb[KCB];
+  };
+  auto blocks_of = [&](int u) {
+    Blocks b;
+    if constexpr (RUN_ON) {
+#pragma unroll
+      for (int c = 0; c < KCB; ++c) {
+        const int i = min(u * KCB + c, nsl * KB2 - 1);
+        b.j[c] = wave + i / KB2 * NW;
+        b.kb[c] = i % KB2;
+      }
+    } else {
+      b.j[0] = wave + (u / nkcb) * NW;
+#pragma unroll
+      for (int c = 0; c < KCB; ++c) b.kb[c] = min((u % nkcb) * KCB + c, KB2 - 1);
+    }
+    return b;
+  };
   auto load_wb = [&](int u, UnitB& x) {
-    const int e = act_ids[wave + (u / nkcb) * NW], kb0 = (u % nkcb) * KCB;
+    const Blocks b = blocks_of(u);
+    int e[NSL];
+#pragma unroll
+    for (int i = 0; i < NSL; ++i) e[i] = act_ids[b.j[i]];
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
 #pragma unroll
       for (int c = 0; c < KCB; ++c) {
-        const size_t blk = ((size_t)e * HT + tl[d]) * KB2 + min(kb0 + c, KB2 - 1);
+        const int ec = e[RUN_ON ? c : 0];
+        const size_t blk = ((size_t)ec * HT + tl[d]) * KB2 + b.kb[c];
         const uint4 z = make_uint4(0, 0, 0, 0);
         if constexpr (a16w4) {
           x.a[d][c][0] = live[d] ? ld_stream16(p.w2 + blk * 1024 + lane * 16) : z;
         } else {
           x.a[d][c][0] = x.a[d][c][a16w4 ? 0 : 1] = z;
           if (live[d]) load_fp8_block(p.w2 + blk * 2048, p.wl, lane, x.a[d][c][0], x.a[d][c][a16w4 ? 0 : 1]);
-          x.sc[d][c] = ((const float*)p.s2)[((size_t)e * (p.H / 128) + tl[d] / 8) * KB2 + min(kb0 + c, KB2 - 1)];
+          x.sc[d][c] = ((const float*)p.s2)[((size_t)ec * (p.H / 128) + tl[d] / 8) * KB2 + b.kb[c]];
         }
       }
-      if constexpr (a16w4) x.sw[d] = e8m0_word(p.s2 + e * e8m0_expert_bytes(p.wl, p.H, p.I), p.wl, p.I, tl[d], kb0, lane);
+      if constexpr (a16w4)
+        x.sw[d] = e8m0_word(p.s2 + e[0] * e8m0_expert_bytes(p.wl, p.H, p.I), p.wl, p.I, tl[d], (u % nkcb) * KCB, lane);
     }
   };
   auto load_mb = [&](int u, UnitB& x) {
-    const int j = wave + (u / nkcb) * NW, kb0 = (u % nkcb) * KCB;
+    const Blocks b = blocks_of(u);
 #pragma unroll
     for (int cg = 0; cg < NCG; ++cg) {
       const int row = cg * 16 + c16;
 #pragma unroll
       for (int c = 0; c < KCB; ++c) {
-        const int kb = min(kb0 + c, KB2 - 1);
+        const int j = b.j[RUN_ON ? c : 0], kb = b.kb[c];
         if constexpr (w8a8) {
           x.bq[c][cg] = load_b_fp8_same(p.mid_q + (size_t)j * p.M * p.I, row, p.M, p.I, kb * 128, g);
           x.ms[c][cg] = row < p.M ? ldp_f32(p.mid_sf + ((size_t)j * p.M + row) * (p.I / 128) + kb) : 0.f;
@@ -1327,12 +1361,13 @@ MK2_DEV void down_rows(const MoeDev& p, int nt, float* red, int* act_ids, float*
           load_b_bf16(p.mid_b + (size_t)j * p.M * p.I, row, p.M, p.I, kb * 128 + 32 * g, x.bb[c][cg]);
         }
       }
-      x.wr[cg] = ldp_f32(p.rw + j * 32 + row);
+#pragma unroll
+      for (int i = 0; i < NSL; ++i) x.wr[i][cg] = ldp_f32(p.rw + b.j[i] * 32 + row);
     }
   };
   f32x4 tb[DT][NCG];  // A16W4: the slot's sums
   auto compute_b = [&](int u, UnitB& x) {
-    const int kb0 = (u % nkcb) * KCB;
+    const int kb0 = RUN_ON ? 0 : (u % nkcb) * KCB;
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
       if (a16w4 && kb0 == 0) {
@@ -1341,14 +1376,14 @@ MK2_DEV void down_rows(const MoeDev& p, int nt, float* red, int* act_ids, float*
       }
 #pragma unroll
       for (int c = 0; c < KCB; ++c) {
-        if (kb0 + c >= KB2) break;
+        if (RUN_ON ? u * KCB + c >= nsl * KB2 : kb0 + c >= KB2) break;
         if constexpr (w8a8) {
           const uint4 lo = x.a[d][c][0], hi = x.a[d][c][a16w4 ? 0 : 1];
           const i32x8 A = {(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
 #pragma unroll
           for (int cg = 0; cg < NCG; ++cg)
             acc[d][cg] += mfma_same<0>(A, x.bq[c][cg], f32x4{0.f, 0.f, 0.f, 0.f}, E8M0_ONE, E8M0_ONE) *
-                          (x.sc[d][c] * x.ms[c][cg] * x.wr[cg]);
+                          (x.sc[d][c] * x.ms[c][cg] * x.wr[RUN_ON ? c : 0][cg]);
         } else if constexpr (a16w4) {
           const float sc = e8m0_to_f32(x.sw[d] >> e8m0_shift(p.wl, tl[d], kb0 + c));
           const uint4 w = x.a[d][c][0];
@@ -1362,12 +1397,12 @@ MK2_DEV void down_rows(const MoeDev& p, int nt, float* red, int* act_ids, float*
                                e4m3x8_to_bf16(hi.z, hi.w)};
 #pragma unroll
           for (int cg = 0; cg < NCG; ++cg)
-            acc[d][cg] += mfma4_bf16(a, x.bb[c][cg], f32x4{0.f, 0.f, 0.f, 0.f}) * (x.sc[d][c] * x.wr[cg]);
+            acc[d][cg] += mfma4_bf16(a, x.bb[c][cg], f32x4{0.f, 0.f, 0.f, 0.f}) * (x.sc[d][c] * x.wr[0][cg]);
         }
       }
       if (a16w4 && kb0 + KCB >= KB2) {
 #pragma unroll
-        for (int cg = 0; cg < NCG; ++cg) acc[d][cg] += tb[d][cg] * x.wr[cg];
+        for (int cg = 0; cg < NCG; ++cg) acc[d][cg] += tb[d][cg] * x.wr[0][cg];
       }
     }
   };

@@ -136,6 +136,33 @@ def test_moe_down_pipeline(fmt, hidden, inter, rows):
     _check(cfg, w, out, logits, ids, wts, norm=True, residual=True)
 
 
+@pytest.mark.parametrize("fmt", ["MXFP4", "A4W4"])
+@pytest.mark.parametrize("hidden, inter, rows", [(7168, 384, 17), (5120, 256, 32), (5120, 128, 20), (2048, 384, 31)])
+def test_moe_compacted_down_tiles(fmt, hidden, inter, rows):
+    """The compacted down in tasks of 32 hidden rows, and of 16, at one k-block a slot and odd
+    numbers of them (6144 takes 24-row tasks)."""
+    from dataclasses import replace
+
+    from sgl_amd_mono.k2 import config as C
+
+    cfg = replace(C.C2_MOE, hidden=hidden, inter=inter, n_experts=64, expert_fmt=getattr(C, "FMT_" + fmt))
+    w, out, logits, ids, wts = _run(cfg, rows, seed=hidden + inter + rows, norm=True, residual=True)
+    _check(cfg, w, out, logits, ids, wts, norm=True, residual=True)
+
+
+@pytest.mark.parametrize("hidden, inter, rows", [(2048, 640, 17), (2048, 128, 32), (3072, 896, 8), (4096, 384, 32), (7168, 384, 5)])
+def test_moe_w8a8_units_across_slots(hidden, inter, rows):
+    """W8A8's units of two k-blocks run on from one slot to the next: odd numbers of blocks a
+    slot, one block a slot, an odd number of them in all on some waves."""
+    from dataclasses import replace
+
+    from sgl_amd_mono.k2 import config as C
+
+    cfg = replace(C.C2_MOE, hidden=hidden, inter=inter, n_experts=64, expert_fmt=C.FMT_W8A8)
+    w, out, logits, ids, wts = _run(cfg, rows, seed=hidden + inter + rows, norm=True, residual=True)
+    _check(cfg, w, out, logits, ids, wts, norm=True, residual=True)
+
+
 def test_moe_mxfp4_norm_residual():
     from sgl_amd_mono.k2 import config as C
 
