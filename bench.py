@@ -172,7 +172,7 @@ def cpu_baseline(layer, reps):
     from refs import CpuLayer
 
     # the host cores this process may use: the OMP_NUM_THREADS share when it is set (a
-    # GPU box gives each GPU a share of its cores), else every core
+    # shared host gives each GPU a share of its cores), else every core
     cores = os.cpu_count() or 1
     share = os.environ.get("OMP_NUM_THREADS", "")
     if share.isdigit() and int(share) > 0:
@@ -195,7 +195,7 @@ def cpu_baseline(layer, reps):
         "cpu_model": cpu_model(),
         "kind": "port",
         "trials_us": [round(t * 1e6, 1) for t in times],
-        "sample": f"1 warm-up + median of {reps} oracle forwards of one configs[4] layer at M={layer.rows} "
+        "sample": f"1 warm-up + median of {reps} oracle forwards of one such layer at M={layer.rows} "
                   f"(f64 index scores over {layer.rows} x 65536 keys); expert dequant {prep:.1f}s outside timing",
     }
 
@@ -360,7 +360,7 @@ def main():
     ap.add_argument("--probes", metavar="MD",
                     help="run the HBM streaming-read and XCD hand-off probes, write a markdown summary and exit")
     ap.add_argument("--standalone", metavar="MD",
-                    help="time configs[0..3], the tail and the front as their own launches; write a table")
+                    help="time the two MoE blocks, the sparse MLA, the indexer, the tail and the front as their own launches; write a table")
     args = ap.parse_args()
     if args.pmc_kernels:
         print(json.dumps(pmc_kernels(args.pmc_kernels, args.calib_bytes), indent=1))
@@ -390,7 +390,7 @@ def main():
     extra = [int(r) for r in args.extra_rows.split(",") if r] if args.extra_rows else []
     extra = [r for r in extra if r != rows]
     # widths above 8 rows are verify steps of 8 requests (8 x 4 draft tokens at 32
-    # rows, as configs[4] names it), built at their width; the decode widths are views
+    # rows, as the workload names it), built at their width; the decode widths are views
     # of one set of layers built at the widest of them
     def is_verify(r):
         return r > 8 and r % 8 == 0
@@ -462,7 +462,7 @@ def main():
         "dtype": "mxfp4+fp8 weights, bf16/fp8 MFMA, f32 accumulate",
         "data": "synthetic (seeded random-init weights ~N(0,0.02), rows ~N(0,1), shuffled pages)",
         "config": {
-            "workload": "configs[4] chained K2 layer: indexer 64x128 FP4 keys ctx 65536 top-2048 -> "
+            "workload": "chained K2 layer: indexer 64x128 FP4 keys ctx 65536 top-2048 -> "
                         "sparse MLA 16 heads 512+64 FP8 KV -> W_UV/W_o -> RMSNorm 1e-6 -> "
                         "MXFP4 MoE 256 experts top-8 inter 256 + FP8 shared",
             "rows": rows,
@@ -585,7 +585,7 @@ def _cpu_time(fn, reps):
 
 
 def standalone(args, dev):
-    """configs[0..3] as their own launches (the MoE block at C1 and C2, sparse MLA at C3,
+    """The layer's parts as their own launches (the MoE block at C1 and C2, sparse MLA at C3,
     the indexer at C4), the tail (C6) and the front (C7), each on one resident copy:
     GPU us (graph replay), algorithmic bytes and the share of 8 TB/s, the oracle's CPU
     us on the same inputs, and the parity of the launch's outputs with the oracle's."""
@@ -648,7 +648,7 @@ def standalone(args, dev):
     sc, tk = op(ns.q, ns.w, ns.cache, ns.cache_scale, ns.page_table, ns.req_ids, ns.ctx_len)
     torch.cuda.synchronize()
     nbytes = 8 * cfg.context * (cfg.dim // 2 + cfg.dim // 32) + 8 * cfg.heads * (cfg.dim + 1) * 2 + 8 * cfg.topk * 4
-    # timed as configs[3] delivers it: the lists, the scores kept inside the launch (the
+    # timed as the layer uses it: the lists, the scores kept inside the launch (the
     # eager call above wrote them for the parity check; the lists are the same bits)
     tk2 = torch.empty_like(tk)
     us, tr = time_graph([lambda: op(ns.q, ns.w, ns.cache, ns.cache_scale, ns.page_table, ns.req_ids, ns.ctx_len,
@@ -697,7 +697,7 @@ def standalone(args, dev):
     ref = fr()
     cpu_us = _cpu_time(fr, reps)
     row("C7 front (K1)", 8, us, tr, wb, cpu_us, f"mla_q rel-L2 {R.rel_l2(cpu(outs[0]).float(), ref['mla_q']):.1e}")
-    lines = [f"# Standalone launches on MI355X: configs[0..3], the tail and the front", "",
+    lines = [f"# Standalone launches on MI355X: the MoE blocks, sparse MLA, the indexer, the tail and the front", "",
              f"Command: `python {shlex.join(sys.argv)}` (sources {sources_digest()[:12]}).", "",
              f"GPU: HIP-graph replay, median of 5 trials. CPU: the oracle on the same inputs, {cores} threads, "
              f"{cpu_model()}, median of {reps} after a warm-up (C4: {max(1, reps // 2)}).", "",

@@ -300,7 +300,7 @@ int mk2_layer_workspace_layout(const mk2_layer_args* args, int64_t* moe_offset);
  * workspace_bytes are ignored; the scratch is a device array of
  * MK2_LAYER_STATIC_SCRATCH_BYTES inside the library, which each GPU the library runs
  * on holds until the process ends.  A shape whose mk2_layer_workspace_bytes exceeds it
- * fails with MK2_ENOSPACE (the configs[4] layer needs about 1.9 MiB a row at context
+ * fails with MK2_ENOSPACE (the benchmark's layer needs about 1.9 MiB a row at context
  * 65536: 60.4 MiB at 32 rows).  Nothing is allocated: each call enqueues a small fill
  * kernel that clears the counters and histograms a launch needs zero and every region
  * of tagged hand-off words (the array keeps the last call's other contents, and calls

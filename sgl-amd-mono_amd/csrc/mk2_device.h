@@ -354,17 +354,7 @@ inline uint32_t wait_ticks_of(int wait_us) {
   return wait_us > 0 ? (uint32_t)wait_us * WAIT_TICKS_PER_US : DEFAULT_WAIT_TICKS;
 }
 
-// ----------------------------------------------------------------- tagged hand-offs
-// A 32-bit value one workgroup hands to another inside a persistent launch can travel
-// with the launch's tag in the same 8-byte word, (tag << 32) | value, stored
-// device-coherently.  The consumer polls the word itself until it carries its
-// launch's tag: one memory round trip, with no store drain on the producer, no
-// counter and no second load.  Tags grow by one a launch and are never 0, so on a
-// workspace whose tagged regions hold only tagged words of earlier launches (a
-// workspace zero-filled before its first launch and used for one shape) a stale word
-// never matches; where the regions may hold other bytes (a scratch array shared by
-// shapes whose layouts differ) the caller clears them before each launch.  Between stream-ordered
-// kernels (one kernel a stage) the stream publishes the words: tag 0, read unchecked.
+// ----------------------------------------------------------------- leaving a launch
 // A launch's word for leaving: workgroups count out in its low bits, and a wait that gives up
 // sets EXIT_FAILED beside them, so the last workgroup's own count-out tells it whether the
 // launch failed.
@@ -385,6 +375,18 @@ MK2_DEV bool launch_exit(int* word, int G, int* lds, bool* failed) {
   *failed = (was & EXIT_FAILED) != 0;
   return (was & ~EXIT_FAILED) == G - 1;
 }
+
+// ----------------------------------------------------------------- tagged hand-offs
+// A 32-bit value one workgroup hands to another inside a persistent launch can travel
+// with the launch's tag in the same 8-byte word, (tag << 32) | value, stored
+// device-coherently.  The consumer polls the word itself until it carries its
+// launch's tag: one memory round trip, with no store drain on the producer, no
+// counter and no second load.  Tags grow by one a launch and are never 0, so on a
+// workspace whose tagged regions hold only tagged words of earlier launches (a
+// workspace zero-filled before its first launch and used for one shape) a stale word
+// never matches; where the regions may hold other bytes (a scratch array shared by
+// shapes whose layouts differ) the caller clears them before each launch.  Between stream-ordered
+// kernels (one kernel a stage) the stream publishes the words: tag 0, read unchecked.
 struct TagPoll {
   uint32_t tag;         // this launch's tag; 0: stream-ordered, no checking
   uint32_t wait_ticks;  // a wait's deadline (WaitClock ticks)

@@ -3,9 +3,9 @@
 //
 // split task (row r, split s): 64 selected positions -> page table -> 576-byte E4M3
 // rows, gathered with 16-byte loads into LDS row-major: the QK operand as it lies, the PV
-// operand (8 keys of a dim a lane) by transposing LDS reads.  S = q . k on bf16 MFMA (E4M3 widens exactly), x (scale_k * sm_scale); a
-// split-local softmax per head; P' = p * scale_k rounded to bf16; O = P' V on bf16
-// MFMA.  The split writes O (unnormalized), its max m and sum l.
+// operand (8 keys of a dim a lane) by transposing LDS reads.  S = q . k on bf16 MFMA (E4M3
+// widens exactly), x (scale_k * sm_scale); a split-local softmax per head; P' = p * scale_k
+// rounded to bf16; O = P' V on bf16 MFMA.  The split writes O (unnormalized), its max m and sum l.
 // merge task (up to 4 rows, head h, half): exact combination of each row's splits ->
 // o_lat (bf16), then o[r][h] = W_UV[h] o_lat on bf16 MFMA, the rows as its columns.
 // oproj task (16 hidden rows): a = bf16(h + W_o o) on bf16 MFMA.

@@ -35,7 +35,7 @@ __global__ __launch_bounds__(MOE_NT) void k_moe_upgate(MoeDev p) {
 
 template <int NCG, int FMT>
 __global__ __launch_bounds__(MOE_NT) void k_moe_down(MoeDev p) {
-  __shared__ float red[(MOE_NT / 64) * 2 * 16 * 32];  // NW * DT * NCG * 256 (DT * NCG <= 2),
+  __shared__ float red[(MOE_NT / 64) * 2 * 16 * 32];  // NW * DT * NCG * 256 (DT * NCG <= 4),
                                                      // or NW * DT * 16 * 32 (compacted rows)
   __shared__ int act_ids[512];
   __shared__ float xres[16 * 2 * 32];

@@ -1499,7 +1499,7 @@ MK2_DEV void down_rows_cmp(const MoeDev& p, int nt, float* red, int* act_ids, fl
   constexpr bool a4 = FMT == MK2_FMT_A4W4;
   down_residual_lds<DT>(p, t, xres, wave);
   // the routed slots (MXFP4): a unit is a batch of B slots (wave + NW * (B * i + u))
-  // over KC k-blocks; units u + 1 and u + 2 (u + 1 alone for 24-row tasks: weights,
+  // over KC k-blocks; units u + 1 and u + 2 (u + 1 alone for tasks of two tiles: weights,
   // mid rows, scales and route weights) are in flight while unit u's MFMAs run
   struct Unit {
     i32x8 a[B][DT][KC];
@@ -1614,7 +1614,7 @@ MK2_DEV void down_rows_cmp(const MoeDev& p, int nt, float* red, int* act_ids, fl
       }
     }
   };
-  // units in flight: 3, or 2 of two tiles each (24-row tasks), within the registers
+  // units in flight: 3, or 2 of two tiles each (24- and 32-row tasks), within the registers
   constexpr int DEPTH = DT == 2 ? 2 : 3;
   Unit x0, x1, x2;
   if (nu > 0) load_w(0, x0);

@@ -13,8 +13,8 @@
 // Wave w owns the k slice [w * hidden / 8, (w + 1) * hidden / 8) of every tile: the
 // normed rows' B operands for that slice (the rows as the MFMA's columns, up to 16 a
 // column group) are built once and stay in registers (part of a second group's in LDS),
-// and the tile's W rows stream through a window of WIN 16-byte loads a lane, each refilled from the same tile or the next one as its MFMA
-// consumes it.  The norm costs no extra pass over the rows: the x fragments a wave
+// and the tile's W rows stream through a window of WIN 16-byte loads a lane, each refilled
+// from the same tile or the next one as its MFMA consumes it.  The norm costs no extra pass over the rows: the x fragments a wave
 // loads for its operands give its slice's sums of squares, which the eight waves
 // combine through LDS; they and the norm weight are loaded ahead of the first window,
 // so the norm runs while the first W bytes are in flight.  A lane (c16, g) loads 16 B

@@ -3,9 +3,9 @@
 The reference fixes one geometry per model in ``glm53/gfx950/config.py:184-197``
 (hidden 6144, kv_lora 512, rope 64, 256 experts, top-8, inter 256 a rank, route
 scale 2.5).  Here each piece of the layer is a frozen dataclass so the same
-kernels serve the FP8 MoE block, the MXFP4 MoE shard,
-sparse MLA, the FP4 indexer and the chained layer
-(configs[4]).
+kernels serve the FP8 MoE block (C1_MOE), the MXFP4 MoE shard (C2_MOE),
+sparse MLA (C3_MLA), the FP4 indexer (C4_INDEXER) and the chained layer
+(C5_LAYER).
 """
 
 from __future__ import annotations
@@ -219,25 +219,25 @@ class TailConfig:
             raise ValueError("eps must be positive")
 
 
-# configs[0]: FP8 MoE block, CPU-runnable
+# FP8 MoE block, CPU-runnable
 C1_MOE = MoEConfig(
     hidden=2048, n_experts=64, top_k=8, inter=768, router=ROUTER_SOFTMAX,
     route_scale=1.0, expert_fmt=FMT_FP8, n_shared=1, shared_inter=768,
 )
-# configs[1]: MXFP4 MoE decode shard (one GPU's share: inter 2048 / 8)
+# MXFP4 MoE decode shard (one GPU's share: inter 2048 / 8)
 C2_MOE = MoEConfig(
     hidden=6144, n_experts=256, top_k=8, inter=256, router=ROUTER_SIGMOID_BIAS,
     route_scale=2.5, expert_fmt=FMT_MXFP4, n_shared=1, shared_inter=256,
 )
-# configs[2]: sparse-MLA decode attention + o_proj
+# sparse-MLA decode attention + o_proj
 C3_MLA = MlaConfig(context=32768)
-# configs[3]: FP4 indexer + exact top-2048
+# FP4 indexer + exact top-2048
 C4_INDEXER = IndexerConfig(context=65536)
-# the chained layer (3 + 4 + 2), one context for indexer and attention
+# the chained layer (C4, C3 and C2), one context for indexer and attention
 C5_LAYER = K2Config(
     mla=replace(C3_MLA, context=65536), indexer=C4_INDEXER, moe=C2_MOE, eps=1e-6
 )
 # the tail after the layer stack (one GPU's share of the LM head)
 C6_TAIL = TailConfig()
-# the layer's front ahead of configs[4] (GLM-5 geometry on one GPU's 16 heads)
+# the layer's front ahead of C5_LAYER (GLM-5 geometry on one GPU's 16 heads)
 C7_FRONT = FrontConfig()

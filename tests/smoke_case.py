@@ -1,5 +1,5 @@
 """The case __graft_entry__.smoke() runs: one persistent launch of the chained K2 layer
-(configs[4] geometry, context cut to 4096 positions) over 2 decode rows, checked
+(the C5_LAYER geometry, context cut to 4096 positions) over 2 decode rows, checked
 piecewise against the CPU oracle (refs.check_layer: top-k lists exact, scores within
 1e-4 of f64, the merged attention, the attention term and the MoE term within rel-L2
 1e-2 of the oracle's, expert ids exact; residual rows ~ N(0, (1/128)^2) so that the

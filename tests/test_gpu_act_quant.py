@@ -241,7 +241,7 @@ def test_moe_activation_bytes_without_norm():
 
 @pytest.mark.parametrize("fmt", ["MXFP4", "W8A8"])
 def test_layer_activation_bytes(fmt):
-    """Inside the persistent layer launch (configs[4] at 8 rows, a shorter context): the
+    """Inside the persistent layer launch (C5_LAYER at 8 rows, a shorter context): the
     router tasks normalize the attention output the launch produced itself."""
     from dataclasses import replace
 

@@ -119,7 +119,7 @@ def test_indexer_config4_full():
 
 
 def test_indexer_config4_verify_width():
-    """configs[3] at the verify width, 32 rows over the full 65536 context: every
+    """C4_INDEXER at the verify width, 32 rows over the full 65536 context: every
     workgroup runs several score chunks and slices of several rows (the standalone
     launch gives slices their tasks in start order by a ticket)."""
     from sgl_amd_mono.k2 import config as C
@@ -193,7 +193,7 @@ def _fp8(cfg):
 
 
 def test_indexer_fp8_cache_config4_full():
-    """configs[3]'s shape with the keys in SGLang's FP8 index pages [pages, 64, 132]."""
+    """C4_INDEXER's shape with the keys in SGLang's FP8 index pages [pages, 64, 132]."""
     from sgl_amd_mono.k2 import config as C
 
     cfg = _fp8(C.C4_INDEXER)
@@ -244,7 +244,7 @@ def _q4(cfg):
 
 @pytest.mark.parametrize("rows", [8, 32])
 def test_indexer_fp4_queries_full_context(rows):
-    """configs[3]'s shape with the queries quantized to MXFP4 in the kernel
+    """C4_INDEXER's shape with the queries quantized to MXFP4 in the kernel
     (KEYS_FP4_Q4, quantize_fp4_indexer_row's rule) and scored on the FP4 x FP4 scaled
     MFMA: scores within 1e-4 of the f64 oracle of the quantized queries (refs.
     index_queries), the list exactly the radix-select list of the kernel's own scores,

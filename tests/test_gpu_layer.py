@@ -75,7 +75,7 @@ def test_layer_small_context_32_rows():
 
 
 def test_layer_verify_width_full_context():
-    """configs[4] at the verify width, 32 rows over the full 65536-position context,
+    """C5_LAYER at the verify width, 32 rows over the full 65536-position context,
     against the oracle: there the persistent launch runs the top-k selects as tasks of
     their own (32 rows x 32 chunks exceed the workgroups) and each workgroup keeps
     several score chunks in LDS for its slices."""
@@ -89,7 +89,7 @@ def test_layer_verify_width_full_context():
 
 @pytest.mark.parametrize("staged", [False, True])
 def test_layer_verify_draft_layout(staged):
-    """configs[4]'s verify step as its config names it: 8 requests x 4 draft tokens
+    """C5_LAYER's verify step: 8 requests x 4 draft tokens
     (32 rows, four a request sharing its index and latent-KV pages, at context lengths
     65533 .. 65536), persistent and staged, against the oracle."""
     from sgl_amd_mono.k2 import config as C
@@ -103,7 +103,7 @@ def test_layer_verify_draft_layout(staged):
 
 @pytest.mark.parametrize("rows", [8, 32])
 def test_layer_fp4_queries(rows):
-    """configs[4] with the FP4 x FP4 index scorer (KEYS_FP4_Q4: the queries quantized to
+    """C5_LAYER with the FP4 x FP4 index scorer (KEYS_FP4_Q4: the queries quantized to
     MXFP4 in the kernel), at the decode and the verify width over the full context,
     against the oracle of the quantized queries."""
     from dataclasses import replace
