@@ -229,10 +229,6 @@ static FrontSteps front_steps(const mk2_front_shape* s) {
 static bool front_persistent_ok(const mk2_front_shape* s) {
   const FrontSteps k = front_steps(s);
   if (s->index_heads > 0 && k.kuw != 1) return false;
-  // (two column groups fit each one's slices: front_prepare plans one pass, the launch's only)
-#define MK2_FP_NARROW(WF, A, C, N) static_assert(A <= GV_KU2 && C <= GV_KU2, "one GEMV pass at 32 rows");
-  MK2_FRONT_PERSISTENT_SHAPES(MK2_FP_NARROW, 0)
-#undef MK2_FP_NARROW
 #define MK2_FP_MATCH(WF, A, C, N) || (k.kua == A && k.kuc == C && k.ns == N)
   return false MK2_FRONT_PERSISTENT_SHAPES(MK2_FP_MATCH, 0);
 #undef MK2_FP_MATCH
@@ -369,8 +365,9 @@ static FrontPDev front_pdev_of(const mk2_front_args* a, const FrontPrep& P) {
   const bool idx = s.index_heads > 0;
   FrontPDev d{};
   d.f = P.f;
-  d.A = P.gA[0]; d.W = P.gW[0]; d.C = P.gC[0];
-  // one round of workgroups for the hidden-input GEMVs: the W_iw workgroups
+  for (int pi = 0; pi < 2; ++pi) { d.A[pi] = P.gA[pi]; d.W[pi] = P.gW[pi]; d.C[pi] = P.gC[pi]; }
+  d.passes = P.passes;
+  // one round of workgroups for a pass's hidden-input GEMVs: the W_iw workgroups
   // first, [W_qkv_a | W_ik] on the rest (a tile's bits do not depend on which
   // workgroup or how many take the tiles)
   d.gridW = idx ? gemv_grid(P.gW[0], P.cus) : 0;

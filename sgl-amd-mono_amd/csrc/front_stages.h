@@ -539,7 +539,6 @@ constexpr int FP_LANES = 8, FP_COPIES = 4, FP_WIDE = FP_LANES * FP_COPIES;
 // GEMV steps and nope 192, block-FP8 weights row-major or in AITER's layout
 enum : int { FRONT_FUSED_NONE = 0, FRONT_FUSED_C7_FP8 = 1, FRONT_FUSED_C7_AITER16 = 2 };
 enum : int {
-  // lines 0 .. 49 are not used: the status word keeps its documented place
   FP_EXIT = 50,                // workgroups finished, and a failed wait (launch_exit)
   FP_STATUS,                   // nonzero once a launch failed; never cleared here
   // wide counters, [FP_WIDE] each
@@ -554,8 +553,8 @@ static_assert(FP_STATUS * FP_LINE * 4 == MK2_FRONT_STATUS_OFFSET, "the status wo
 
 struct FrontPDev {
   FrontDev f;
-  GemvDev A, W, C;  // one pass: every shape's slices take two column groups
-  int gridA, gridW, gridC, nheads;
+  GemvDev A[2], W[2], C[2];  // by pass: the rows the engine takes at once (16 or 32)
+  int passes, gridA, gridW, gridC, nheads;
   const bf16_t* x;
   const bf16_t* g_in;
   bf16_t* x_n;
@@ -644,34 +643,36 @@ MK2_DEV bool front_walk(const FrontPDev& p, FrontLds& S, int* seen) {
     fp_signal(p, FP_NORM, t);
   }
   FP_NEXT(M);
-  // 1. the hidden-input GEMVs: [W_qkv_a | W_ik], then W_iw
+  // 1. the hidden-input GEMVs, per pass: [W_qkv_a | W_ik], then W_iw
   const int nA = p.gridA + p.gridW;
-  FP_TASKS(t, nA) {
+  FP_TASKS(t, p.passes * nA) {
+    const int pass = t / nA, u = t % nA;
     auto w = [&] { return fp_wait(p, seen, 0, FP_NORM, M); };
-    const bool ok = t < p.gridA ? gemv_run<KUA, WF, NCG>(p.A, t, p.gridA, S.gemv, w)
-                                : gemv_run<1, MK2_WFMT_BF16, NCG>(p.W, t - p.gridA, p.gridW, S.gemv, w);
+    const bool ok = u < p.gridA ? gemv_run<KUA, WF, NCG>(p.A[pass], u, p.gridA, S.gemv, w)
+                                : gemv_run<1, MK2_WFMT_BF16, NCG>(p.W[pass], u - p.gridA, p.gridW, S.gemv, w);
     if (!ok) return false;
     fp_signal(p, FP_A, t);
   }
-  FP_NEXT(nA);
+  FP_NEXT(p.passes * nA);
   // 2. the per-row stage
   const int nR = (p.f.ih ? 3 : 2) * M;
   FP_TASKS(t, nR) {
-    if (!fp_wait(p, seen, 1, FP_A, nA)) return false;
+    if (!fp_wait(p, seen, 1, FP_A, p.passes * nA)) return false;
     front_rows_task(p.f, t, S.rows.sh, S.rows.kvv);
     fp_signal(p, FP_ROWS, t);
   }
   FP_NEXT(nR);
   // 3. the q_an-input GEMVs
-  FP_TASKS(t, p.gridC) {
-    if (!gemv_run<KUC, WF, NCG>(p.C, t, p.gridC, S.gemv, [&] { return fp_wait(p, seen, 2, FP_ROWS, nR); }))
+  FP_TASKS(t, p.passes * p.gridC) {
+    const int pass = t / p.gridC, u = t % p.gridC;
+    if (!gemv_run<KUC, WF, NCG>(p.C[pass], u, p.gridC, S.gemv, [&] { return fp_wait(p, seen, 2, FP_ROWS, nR); }))
       return false;
     fp_signal(p, FP_C, t);
   }
-  FP_NEXT(p.gridC);
+  FP_NEXT(p.passes * p.gridC);
   // 4. the per-head stage
   FP_TASKS(t, p.nheads) {
-    if (!front_heads_task<NS>(p.f, t, S.qn, [&] { return fp_wait(p, seen, 3, FP_C, p.gridC); }))
+    if (!front_heads_task<NS>(p.f, t, S.qn, [&] { return fp_wait(p, seen, 3, FP_C, p.passes * p.gridC); }))
       return false;
     if constexpr (HEADS) fp_signal(p, FP_HEADS, t);
     else __syncthreads();  // this workgroup's next head task rewrites qn
