@@ -229,6 +229,10 @@ static FrontSteps front_steps(const mk2_front_shape* s) {
 static bool front_persistent_ok(const mk2_front_shape* s) {
   const FrontSteps k = front_steps(s);
   if (s->index_heads > 0 && k.kuw != 1) return false;
+  // (two column groups fit each one's slices: front_prepare plans one pass)
+#define MK2_FP_NARROW(WF, A, C, N) static_assert(A <= GV_KU2 && C <= GV_KU2, "one GEMV pass at 32 rows");
+  MK2_FRONT_PERSISTENT_SHAPES(MK2_FP_NARROW, 0)
+#undef MK2_FP_NARROW
 #define MK2_FP_MATCH(WF, A, C, N) || (k.kua == A && k.kuc == C && k.ns == N)
   return false MK2_FRONT_PERSISTENT_SHAPES(MK2_FP_MATCH, 0);
 #undef MK2_FP_MATCH
