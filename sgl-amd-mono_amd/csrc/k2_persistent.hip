@@ -98,7 +98,7 @@ static_assert(sizeof(FrontLds) <= sizeof(TopkLds), "the front's LDS fits the lay
 // pointers and sizes it uses as it starts (scalar cache hits).  With one view of the
 // arguments for the whole walk they were loaded up front and lived, spilled to vector lanes,
 // through every stage: 205 of them at 32 rows and 264 at 8 of the A8W4 layer, with a view a
-// stage 96 and 116 (vector spills at 32 rows 38 -> 24), and the layer 225.7 -> 214.4 us at
+// stage 100 and 116 (vector spills at 32 rows 38 -> 24), and the layer 225.7 -> 214.4 us at
 // 32 rows, the indexer's launch 23.4 -> 22.9 at 8 x 65536.
 // A kernel takes the pointer in its own body, K2_ARGS: in a function that is not inlined
 // into it the builtin is 0.

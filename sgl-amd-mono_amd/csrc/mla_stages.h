@@ -123,8 +123,10 @@ MK2_DEV bool mla_split_tasks(const MlaDev& p, int t0, int t1, int iters, MlaSpli
     }
     return (int)pair_value(w);
   };
-  // (the page's load has no use here to wait for)
-  auto page_of = [&](int t, int pos) { return mla_page(p.pt, p.req, t / p.nsplit, p.stride, pos); };
+  // (the page's load has no use here to wait for; its row's line is taken ahead of the poll:
+  // behind it the 8-row layer was 1 us slower)
+  auto line_of = [&](int t) { return mla_line(p.req, t / p.nsplit, p.stride); };
+  auto page_of = [&](ptrdiff_t line, int pos) { return mla_page(p.pt, line, p.stride, pos); };
   auto cache_row = [&](int pos, int page) { return mla_cache_row(pos, page, p.stride); };
   // gather: 16-byte piece i % 36 of key i / 36; every load of a thread is issued at once,
   // the rows' scales ahead of them
@@ -152,8 +154,9 @@ MK2_DEV bool mla_split_tasks(const MlaDev& p, int t0, int t1, int iters, MlaSpli
   if (wave == 0) {
     bool bad = false;
     if (any) {
+      const ptrdiff_t line = line_of(t0);
       const int pos = list_poll(t0, list_word(t0), &bad);
-      L.row[0][lane] = cache_row(pos, page_of(t0, pos));
+      L.row[0][lane] = cache_row(pos, page_of(line, pos));
     }
     if (lane == 0) L.bad = bad;  // wave-uniform
   }
@@ -162,8 +165,9 @@ MK2_DEV bool mla_split_tasks(const MlaDev& p, int t0, int t1, int iters, MlaSpli
   __syncthreads();
   if (failed()) return false;
   if (ahead) {
+    const ptrdiff_t line = line_of(t0 + 1);
     apos = list_poll(t0 + 1, aw, &abad);
-    apage = page_of(t0 + 1, apos);
+    apage = page_of(line, apos);
     if (t0 + 2 < t1) aw = list_word(t0 + 2);
   }
   if (any) {
@@ -197,8 +201,9 @@ MK2_DEV bool mla_split_tasks(const MlaDev& p, int t0, int t1, int iters, MlaSpli
       // the pages of the task after it and the list words of the one after that go out ahead
       // of the gather: behind it they would hold this wave, and so the barriers, to its end
       if (ahead && t + 2 < t1) {
+        const ptrdiff_t line = line_of(t + 2);
         apos = list_poll(t + 2, aw, &abad);
-        apage = page_of(t + 2, apos);
+        apage = page_of(line, apos);
         if (t + 3 < t1) aw = list_word(t + 3);
       }
       gather(L.row[par ^ 1]);

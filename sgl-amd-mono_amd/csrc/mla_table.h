@@ -15,12 +15,14 @@ namespace mk2 {
 // whether a position is one of the table's (a list holds -1 for an unused entry)
 MK2_HOST_DEV bool mla_on_page(int pos, int stride) { return pos >= 0 && pos < stride * 64; }
 
-// row r's page-table entry for a position.  An unused one reads the table's first entry,
-// whatever the row's request id is: a pad row, whose list is all unused, need not name a
-// request of the table.  (A read and no branch, which would wait for it.)
-MK2_HOST_DEV int mla_page(const int32_t* pt, const int32_t* req, int r, int stride, int pos) {
-  const ptrdiff_t at = (ptrdiff_t)req[r] * stride + (pos >> 6);
-  return pt[mla_on_page(pos, stride) ? at : 0];
+// where row r's line of the page table starts.  A pad row, whose list is all unused, need not
+// name a request of the table.
+MK2_HOST_DEV ptrdiff_t mla_line(const int32_t* req, int r, int stride) { return (ptrdiff_t)req[r] * stride; }
+
+// the page-table entry of a position.  An unused one reads the table's first entry, whatever
+// its row's line is (a read and no branch, which would wait for it).
+MK2_HOST_DEV int mla_page(const int32_t* pt, ptrdiff_t line, int stride, int pos) {
+  return pt[mla_on_page(pos, stride) ? line + (pos >> 6) : 0];
 }
 
 MK2_HOST_DEV int mla_cache_row(int pos, int page, int stride) {

@@ -29,7 +29,7 @@ int main() {
     for (int pos : {-1, 0, 63, 64, 16383, 16384, INT32_MAX, INT32_MIN}) {
       const bool used = pos >= 0 && pos < stride * 64;
       if (r >= 2 && used) continue;
-      const int row = mk2::mla_cache_row(pos, mk2::mla_page(pt, req, r, stride, pos), stride);
+      const int row = mk2::mla_cache_row(pos, mk2::mla_page(pt, mk2::mla_line(req, r, stride), stride, pos), stride);
       const int want = used ? (5000 + req[r] * stride + pos / 64) * 64 + pos % 64 : -1;
       if (row != want) return printf("row %d pos %d: %d, not %d\n", r, pos, row, want), 1;
     }
