@@ -85,7 +85,7 @@ size_t moe_carve(const mk2_moe_shape* s, void* base, MoeDev* d) {
   // up/gate chunks: 128 intermediate rows for W8A8 (its mid is quantized per 128), 64
   // for E2M1 weights up to 16 rows, else 32
   t.UC = fmt == MK2_FMT_W8A8 ? 128 : (w_fp4(fmt) && M <= 16 && I % 64 == 0) ? 64 : 32;
-  t.DR = down_task_rows(H);
+  t.DR = down_task_rows(H, M, fmt);
   t.ssp = c.take<float>((size_t)(H / 16) * M);
   t.xn = c.take<bf16_t>((size_t)M * H);
   t.xq = c.take<uint8_t>((size_t)M * H);

@@ -1704,7 +1704,12 @@ MK2_DEV void down_rows_cmp(const MoeDev& p, int nt, float* red, int* act_ids, fl
 // worth of mid loads and hand-offs.  2048, 3072 and 4096 -> 16 (128, 192, 256 tasks), 6144 ->
 // 24 (256), 7168 -> 32 (224).  A8W4 at 2048, 8 rows (128 experts of 768): 62.0 -> 56.4 us in
 // 16-row tasks instead of 32; 8-row tasks took 59.3 (half-empty tiles, twice the mid loads).
-inline int down_task_rows(int H) {
+// The scaled-MFMA modes at up to 4 rows take 32 where 24 does not fit whole tiles into H: with
+// few slots a wave what counts is the loads it has in flight, and two tiles have twice one's
+// (hidden 4096, experts of 256, in 32-row tasks / in 16: A8W4 at 1 row 25.1 / 26.3 us, at 4
+// rows 31.6 / 31.9, at 5 rows 33.3 / 33.0; A4W4 at 1 row 24.4 / 26.0, at 4 rows 30.4 / 31.4).
+inline int down_task_rows(int H, int M, int fmt) {
+  if (M <= 4 && (fmt == MK2_FMT_MXFP4 || fmt == MK2_FMT_A4W4) && H % 48 && H % 32 == 0) return 32;
   int best = 16, cost = 1 << 30;
   for (const int rows : {32, 24, 16}) {
     if (H % rows) continue;

@@ -122,6 +122,20 @@ def test_moe_mxfp4_down_tiles(hidden):
     _check(cfg, w, out, logits, ids, wts, norm=True, residual=True)
 
 
+@pytest.mark.parametrize("fmt", ["MXFP4", "A4W4"])
+@pytest.mark.parametrize("hidden, rows", [(512, 1), (2048, 4), (4096, 1), (4096, 5)])
+def test_moe_narrow_down_tiles(fmt, hidden, rows):
+    """Up to 4 rows the scaled-MFMA downs take 32 hidden rows a task, at 5 the rule of the
+    wider calls."""
+    from dataclasses import replace
+
+    from sgl_amd_mono.k2 import config as C
+
+    cfg = replace(C.C2_MOE, hidden=hidden, n_experts=64, expert_fmt=getattr(C, "FMT_" + fmt))
+    w, out, logits, ids, wts = _run(cfg, rows, seed=hidden + rows, norm=True, residual=True)
+    _check(cfg, w, out, logits, ids, wts, norm=True, residual=True)
+
+
 @pytest.mark.parametrize("fmt", ["FP8", "W8A8", "A16W4"])
 @pytest.mark.parametrize("hidden, inter, rows", [(6144, 128, 3), (2048, 384, 17), (7168, 384, 20), (6144, 256, 16)])
 def test_moe_down_pipeline(fmt, hidden, inter, rows):
